@@ -87,7 +87,9 @@ int lsmhip_weno5_stage_reinit(LSMLIB_REAL *phi_out, const LSMLIB_REAL *phi_stage
  * three arrays on gb over box b. */
 int lsmhip_deform_velocity_fill(LSMLIB_REAL *vel_x, LSMLIB_REAL *vel_y, LSMLIB_REAL *vel_z, LSMHIP_BOX_ARGS(gb),
                                 LSMHIP_BOX_ARGS(b), const LSMLIB_REAL *const *tabs, LSMLIB_REAL c);
-/* k planes a fused-stage block marches through (default 64). */
+/* k planes a fused-stage block marches through; 0 (the default) takes them
+ * from the grid's size.  FP64 results do not depend on it; FP32 ones only in
+ * which products the compiler contracts. */
 void lsmhip_set_fused_kchunk(int planes);
 /* FP32 library: 1 (default) selects the stage kernels that form a WENO5
  * window per cell, 2 the kernels that form each position's WENO5 terms once and

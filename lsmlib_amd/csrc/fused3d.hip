@@ -887,7 +887,31 @@ bool launch_rhs(int stage, const FusedArgs& a, int nblocks) {
   return true;
 }
 
-int g_kchunk = 64;
+// Planes per chunk: a value set by lsmhip_set_fused_kchunk, or 0 for the rule below.
+int g_kchunk = 0;
+
+// Planes a block marches through.  A chunk costs its planes plus a fixed part
+// (filling the z window, the launch of the block), so long chunks are cheaper
+// per plane; but a grid has to be cut into enough blocks to fill 256 CUs with
+// 2-4 resident blocks each, and into enough more that the last round of blocks
+// does not leave the chip idle.  The rule: chunks of at most 32 planes, shorter
+// where they would give fewer than kBlocks blocks, evened out over the planes.
+// Measured (stage 2, us; chunks of 64 planes -> this rule): FP32 advection 64^3
+// 71.6 -> 5.7, 128^3 71 -> 16, 256^3 103 -> 82, 512^3 680 -> 672; FP64 advection
+// 64^3 201 -> 10, 128^3 160 -> 45, 203 x 149 x 97 212 -> 92, 512^3 2193 -> 2192.
+// FP64 blocks run 2-3 times longer per plane and fewer fit a CU, so the tail of
+// a short last round weighs more: twice the blocks.  Over 14 sizes from 32^3 to
+// 512^3 the rule is within 3 % (mean) of the best chunk of a sweep; 16 and 64
+// planes at most, and 512 blocks, were 1-4 % behind it.
+int chunk_planes(const Box& fb, int nti, int ntj) {
+  constexpr long long kBlocks = sizeof(real_t) == 4 ? 1024 : 2048;
+  constexpr int kMost = 32;
+  const int nz = fb.nz();
+  const long long fit = (long long)nti * ntj * nz / kBlocks;
+  const int kc = fit < 1 ? 1 : fit > kMost ? kMost : (int)fit;
+  const int chunks = (nz + kc - 1) / kc;
+  return (nz + chunks - 1) / chunks;
+}
 
 int run(const char* who, FusedArgs a, int stage) {
   if (a.fb.empty()) return 0;
@@ -899,9 +923,9 @@ int run(const char* who, FusedArgs a, int stage) {
   }
   a.sy = a.gb.nx();
   a.sz = a.gb.nx() * a.gb.ny();
-  a.kc = g_kchunk;
   a.nti = (a.fb.nx() + TX - 1) / TX;
   a.ntj = (a.fb.ny() + TY - 1) / TY;
+  a.kc = g_kchunk > 0 ? g_kchunk : chunk_planes(a.fb, a.nti, a.ntj);
   a.ntk = (a.fb.nz() + a.kc - 1) / a.kc;
   const long long nt = (long long)a.nti * a.ntj * a.ntk;
   const int per = (int)((nt + 7) / 8);
@@ -1045,7 +1069,7 @@ LSMHIP_EXPORT int lsmhip_deform_velocity_fill(real_t* vx, real_t* vy, real_t* vz
   return 0;
 }
 
-LSMHIP_EXPORT void lsmhip_set_fused_kchunk(int kc) { g_kchunk = kc < 1 ? 1 : kc; }
+LSMHIP_EXPORT void lsmhip_set_fused_kchunk(int kc) { g_kchunk = kc < 0 ? 0 : kc; }
 
 // FP32 build: 1 (default) selects the stage kernels that form a WENO5 window
 // per cell, 2 the kernels that share each position's WENO5 terms between

@@ -140,3 +140,47 @@ def test_fused_fp32_close_to_fp64(solvers, kind, kernels):
     assert select(prev) == kernels
     # FP32 storage and arithmetic: relative-to-O(1) errors of a few ulp per step
     assert np.abs(res[0] - res[1]).max() < 2e-5
+
+
+# Tiles of 64 x 8 cells and chunks of planes: single cells, one cell past a tile, and grids that the chunk rule cuts
+# into one plane, a few planes and its longest chunks (with a shorter last one).
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 2, 5), (64, 8, 4), (65, 9, 7), (72, 17, 33), (130, 70, 101), (520, 270, 66)])
+@pytest.mark.parametrize("kind", ["normal", "reinit", "advect"])
+def test_stage_does_not_depend_on_the_chunks(prec, n, kind):
+    """The chunks that the library takes from the grid's size against chunks of 64 planes: the same bits in FP64.  In
+    FP32 the advection kernel's unrolled planes and its last ones may contract different products: each derivative,
+    bounded by the largest difference, moves by some 50 roundings (a reconstruction's operations, its weights moving
+    four times as much as their terms), dt |v| / dx <= 0.2 times that enters, over three axes."""
+    import torch
+    from lsmlib_amd.solver import Grid, Solver
+    g = Grid(n, hi=tuple(0.05 * v for v in n))
+    s = Solver(g, prec)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    us, uc = (torch.randn(g.shape, dtype=s.dtype, device="cuda", generator=gen) for _ in range(2))
+    dt = 0.1 * g.dx[0]
+
+    def run(stage):
+        out = s.field()
+        if kind == "normal":
+            s.stage_normal(out, us, uc, stage, dt, vn=-0.8)
+        elif kind == "reinit":
+            s.stage_reinit(out, us, uc, stage, dt)
+        else:
+            s.stage_deform(out, us, uc, stage, dt, 0.7)
+        return out
+
+    chunk = s.lib.cdll.lsmhip_set_fused_kchunk
+    for stage in (1, 2, 3):
+        a = run(stage)
+        chunk(64)
+        try:
+            b = run(stage)
+        finally:
+            chunk(0)
+        assert torch.isfinite(a).all()
+        if prec == "f64":
+            assert torch.equal(a, b), "stage %d" % stage
+        else:
+            bound = 3 * 0.2 * 4 * 50 * 2.0 ** -24 * 2 * float(us.abs().max())
+            assert float((a - b).abs().max()) <= bound, "stage %d" % stage
