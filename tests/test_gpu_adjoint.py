@@ -95,6 +95,53 @@ def test_stage_adjoint_matches_torch_autograd(stage):
         assert rel(g.interior(s.host(lam_uc)), guc.numpy()) < 1e-12
 
 
+# The marches: waves of 58 targets (with x) and 64 cells, four columns a block, chunks of 8 to 64 targets along j and k,
+# eight flags at a time; the smallest periodic grid, one past each, and lam_out empty, sparse and full.
+@pytest.mark.parametrize("n", [(3, 3, 3), (52, 5, 4), (53, 7, 61), (65, 66, 3), (117, 4, 130)])
+@pytest.mark.parametrize("share", [0.0, 0.02, 1.0])
+def test_stage_adjoint_over_tiles_and_sparse_gradients(n, share):
+    """Against torch autograd on the CPU, as above (the same tolerance), and into lam_out itself (the route of
+    overlapping arrays): lam_out + what the stage adds elsewhere."""
+    import torch
+    from lsmlib_amd.adjoint import NormalMotionAdjoint
+    from lsmlib_amd.solver import Grid
+    g = Grid(n, hi=(1.0, 1.1, 0.9))
+    eng = NormalMotionAdjoint(g, "f64", steps=1)
+    s = eng.solver
+    rng = np.random.default_rng(n[0])
+    shape = (n[2], n[1], n[0])
+    us, uc, w = (rng.standard_normal(shape) for _ in range(3))
+    V = np.where(rng.random(shape) < 0.5, -1.0, 1.0) * (0.5 + rng.random(shape))
+    lam_out = np.where(rng.random(shape) < share, w, 0.0)
+    dt, stage = 0.2 * min(g.dx), 3
+    tus, tuc, tV = (torch.tensor(a, dtype=torch.float64, requires_grad=True) for a in (us, uc, V))
+    out = _torch_stage(tus, tuc, tV, dt, g.dx, stage)
+    want = [a.numpy() for a in torch.autograd.grad((out * torch.tensor(lam_out)).sum(), (tus, tuc, tV))]
+
+    def ghost(a):
+        full = np.zeros(g.shape)
+        g.interior(full)[...] = a
+        return s.field(full)
+
+    d_us, d_V, d_lam = ghost(us), ghost(V), ghost(lam_out)
+    s.fill_ghosts(d_us)
+    lam_us, lam_uc, lam_v = s.field(), s.field(), s.field()
+    eng._stage_adjoint(lam_us, lam_uc, lam_v, d_lam, d_us, stage, d_V, dt)
+    shared = d_lam.clone()
+    eng._stage_adjoint(shared, None, None, shared, d_us, stage, d_V, dt)
+    s.lib.check()
+    scale = max(float(lam_us.abs().max()), 1e-300)
+    assert float((shared - d_lam - lam_us).abs().max()) <= 1e-12 * scale
+    eng._fold_ghosts(lam_us)
+    s.lib.check()
+    inner = torch.zeros(g.shape, dtype=torch.bool, device="cuda")
+    inner[3:-3, 3:-3, 3:-3] = True
+    assert not lam_us[~inner].any()
+    for got, ref in zip((lam_us, lam_uc, lam_v), want):
+        d = np.abs(g.interior(s.host(got)) - ref).max()
+        assert d <= 1e-10 * np.abs(ref).max()
+
+
 def test_two_forward_runs_on_one_engine_keep_their_own_gradients():
     """Two Evolve nodes on one engine before a single backward (a summed loss)
     give, for each speed and phi0, the gradients of separate runs: each node
