@@ -115,7 +115,7 @@ __device__ __forceinline__ void halo_pos(int h, int& px, int& py) {
 }
 
 template <int RHS, int STAGE>
-__global__ void __launch_bounds__(TX* TY) fused_stage_kernel(FusedArgs a) {
+__global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_stage_kernel(FusedArgs a) {
   __shared__ real_t plane[PLANE];
   const int tid = threadIdx.y * TX + threadIdx.x;
 

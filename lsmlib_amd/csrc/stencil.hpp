@@ -10,31 +10,69 @@
 namespace lsmhip {
 namespace stencil {
 
+// n / x and 1 / x in FP64 as the compiler forms them (the hardware's reciprocal
+// estimate, two Newton-Raphson steps, and Markstein's correction of the quotient
+// by its exact remainder), without the scaling and fix-up of operands near the
+// ends of the exponent range: the same operations on the same operands, so the
+// same correctly rounded result, for x and n / x between 2^-700 and 2^700.
+__device__ __forceinline__ double rcp_steps(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double div_in_range(double n, double x) {
+  const double r = rcp_steps(x), q = n * r;
+  return __builtin_fma(__builtin_fma(-x, q, n), r, q);
+}
+__device__ __forceinline__ double inv_in_range(double x) {
+  const double r = rcp_steps(x);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+
 // One HJ-WENO5 reconstruction from five scaled differences, in the order of
 // src/toolbox/lsm_spatial_derivatives3d.f.in:1296-1323.  tiny is the additive
 // term of eps: the templated 1e-36, or the literal 1e-35 of the 2D narrow-band
 // routine (lsm_spatial_derivatives2d_local.f.in:892).
-template <class T>
-__device__ __forceinline__ T weno5(T v1, T v2, T v3, T v4, T v5, T tiny = T(1.e-36)) {
-  const T one_third = T(1.0 / 3.0), seven_sixths = T(7.0 / 6.0), eleven_sixths = T(11.0 / 6.0);
-  const T one_sixth = T(1.0 / 6.0), five_sixths = T(5.0 / 6.0);
-  const T thirteen_twelfths = T(13.0 / 12.0), one_fourth = T(0.25);
-  T m = v1 * v1;
-  m = v2 * v2 > m ? v2 * v2 : m;
-  m = v3 * v3 > m ? v3 * v3 : m;
-  m = v4 * v4 > m ? v4 * v4 : m;
-  m = v5 * v5 > m ? v5 * v5 : m;
-  const T eps = T(1e-6) * m + tiny;
-  const T p1 = one_third * v1 - seven_sixths * v2 + eleven_sixths * v3;
-  const T p2 = -(one_sixth * v2) + five_sixths * v3 + one_third * v4;
-  const T p3 = one_third * v3 + five_sixths * v4 - one_sixth * v5;
-  const T S1 = thirteen_twelfths * sq(v1 - T(2) * v2 + v3) + one_fourth * sq(v1 - T(4) * v2 + T(3) * v3);
-  const T S2 = thirteen_twelfths * sq(v2 - T(2) * v3 + v4) + one_fourth * sq(v2 - v4);
-  const T S3 = thirteen_twelfths * sq(v3 - T(2) * v4 + v5) + one_fourth * sq(T(3) * v3 - T(4) * v4 + v5);
-  T a1 = T(0.1) / sq(S1 + eps);
-  T a2 = T(0.6) / sq(S2 + eps);
-  T a3 = T(0.3) / sq(S3 + eps);
-  const T inv = T(1.0) / (a1 + a2 + a3);
+//
+// Every rounding is the reference's.  Products by 2, 4 and 0.25 are exact, so an
+// FMA in their place rounds what the sum rounds (a product by 0.25 that falls
+// below the normal range is lost beside eps >= 1e-36 either way); max v^2 is
+// (max |v|)^2, as rounding is monotonic.  With max v^2 < 2^200 the denominators
+// lie between 2^-240 and 2^412 and the divisions need no scaling; a wave with a
+// larger value (or a NaN in the maximum) takes the plain divisions.  About 93
+// VALU instructions instead of 127, without the scaling's slow ones.
+__device__ __forceinline__ double weno5(double v1, double v2, double v3, double v4, double v5, double tiny = 1.e-36) {
+  const double one_third = 1.0 / 3.0, seven_sixths = 7.0 / 6.0, eleven_sixths = 11.0 / 6.0;
+  const double one_sixth = 1.0 / 6.0, five_sixths = 5.0 / 6.0;
+  const double thirteen_twelfths = 13.0 / 12.0;
+  const double am = __builtin_fmax(
+      __builtin_fmax(__builtin_fmax(__builtin_fmax(__builtin_fabs(v1), __builtin_fabs(v2)), __builtin_fabs(v3)),
+                     __builtin_fabs(v4)),
+      __builtin_fabs(v5));
+  const double m = am * am;
+  const double eps = 1e-6 * m + tiny;
+  const double p1 = one_third * v1 - seven_sixths * v2 + eleven_sixths * v3;
+  const double p2 = -(one_sixth * v2) + five_sixths * v3 + one_third * v4;
+  const double p3 = one_third * v3 + five_sixths * v4 - one_sixth * v5;
+  const double t3 = 3.0 * v3;
+  const double c1 = __builtin_fma(-2.0, v2, v1) + v3, d1 = __builtin_fma(-4.0, v2, v1) + t3;
+  const double c2 = __builtin_fma(-2.0, v3, v2) + v4, d2 = v2 - v4;
+  const double c3 = __builtin_fma(-2.0, v4, v3) + v5, d3 = __builtin_fma(-4.0, v4, t3) + v5;
+  const double x1 = sq(__builtin_fma(0.25, sq(d1), thirteen_twelfths * sq(c1)) + eps);
+  const double x2 = sq(__builtin_fma(0.25, sq(d2), thirteen_twelfths * sq(c2)) + eps);
+  const double x3 = sq(__builtin_fma(0.25, sq(d3), thirteen_twelfths * sq(c3)) + eps);
+  double a1, a2, a3, inv;
+  if (__builtin_amdgcn_ballot_w64(!(m < 0x1p200)) == 0) {
+    a1 = div_in_range(0.1, x1);
+    a2 = div_in_range(0.6, x2);
+    a3 = div_in_range(0.3, x3);
+    inv = inv_in_range(a1 + a2 + a3);
+  } else {
+    a1 = 0.1 / x1;
+    a2 = 0.6 / x2;
+    a3 = 0.3 / x3;
+    inv = 1.0 / (a1 + a2 + a3);
+  }
   a1 = a1 * inv;
   a2 = a2 * inv;
   a3 = a3 * inv;
