@@ -32,15 +32,17 @@ struct PlusMinusLine {
   real_t inv[3];
   struct In {};
   __device__ In load(int, int, int) const { return In{}; }
-  __device__ void store(int i, int j, int k, const real_t (&fx)[7], const real_t (&fy)[7], const real_t (&fz)[7],
-                        const In&) const {
+  __device__ void store(int i, int j, int k, bool active, const real_t (&fx)[7], const real_t (&fy)[7],
+                        const real_t (&fz)[7], const In&) const {
     const real_t* f[3] = {fx, fy, fz};
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       real_t p, m;
       stencil::plus_minus<ORDER>(f[d], inv[d], p, m);
-      plus.o[d](i, j, k) = p;
-      minus.o[d](i, j, k) = m;
+      if (active) {
+        plus.o[d](i, j, k) = p;
+        minus.o[d](i, j, k) = m;
+      }
     }
   }
 };
@@ -53,13 +55,15 @@ struct UpwindLine {
     real_t v[3];
   };
   __device__ In load(int i, int j, int k) const { return In{{vx(i, j, k), vy(i, j, k), vz(i, j, k)}}; }
-  __device__ void store(int i, int j, int k, const real_t (&fx)[7], const real_t (&fy)[7], const real_t (&fz)[7],
-                        const In& in) const {
+  __device__ void store(int i, int j, int k, bool active, const real_t (&fx)[7], const real_t (&fy)[7],
+                        const real_t (&fz)[7], const In& in) const {
     const real_t* f[3] = {fx, fy, fz};
 #pragma unroll
-    for (int d = 0; d < 3; d++)
-      out.o[d](i, j, k) =
+    for (int d = 0; d < 3; d++) {
+      const real_t r =
           fabs(in.v[d]) < kZeroTol ? real_t(0) : stencil::upwind<ORDER>(f[d], inv[d], in.v[d] > real_t(0));
+      if (active) out.o[d](i, j, k) = r;
+    }
   }
 };
 
@@ -92,8 +96,9 @@ struct Central4Line {
   real_t r[3];
   struct In {};
   __device__ In load(int, int, int) const { return In{}; }
-  __device__ void store(int i, int j, int k, const real_t (&fx)[7], const real_t (&fy)[7], const real_t (&fz)[7],
-                        const In&) const {
+  __device__ void store(int i, int j, int k, bool active, const real_t (&fx)[7], const real_t (&fy)[7],
+                        const real_t (&fz)[7], const In&) const {
+    if (!active) return;
     const real_t e = real_t(8);
     const real_t* f[3] = {fx, fy, fz};
 #pragma unroll

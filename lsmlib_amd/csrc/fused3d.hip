@@ -62,12 +62,21 @@ __device__ __forceinline__ void deform_velocity(const real_t* const ta[3], const
 
 // WENO5 derivatives of the fused stage: the reference's operation order in
 // FP64 (bitwise equal to the drop-in chain), the rearranged FP32 forms in FP32.
+// (stencil::plus_minus<5>, with the minus window's inputs tied to the plus
+// derivative: formed side by side the two windows need 140 registers and leave
+// one block to a CU instead of two)
 __device__ __forceinline__ void weno_pm(const double f[7], double inv, double& p, double& m) {
-  stencil::plus_minus<5>(f, inv, p, m);
+  double v[6];
+#pragma unroll
+  for (int s = 0; s < 6; s++) v[s] = (f[s + 1] - f[s]) * inv;
+  p = stencil::weno5(v[5], v[4], v[3], v[2], v[1]);
+  asm volatile("" : "+v"(p), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]));
+  m = stencil::weno5(v[0], v[1], v[2], v[3], v[4]);
 }
 __device__ __forceinline__ void weno_pm(const float f[7], float inv, float& p, float& m) {
   stencil::fastf::plus_minus(f, inv, p, m);
 }
+
 __device__ __forceinline__ double weno_up(const double f[7], double inv, bool vpos) {
   return stencil::upwind<5>(f, inv, vpos);
 }
@@ -132,6 +141,13 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
   const int i = i0 + threadIdx.x, j = j0 + threadIdx.y;
   const Box gb = a.gb;
   const bool active = i <= a.fb.ihi && j <= a.fb.jhi;
+  // FP64: the lanes past a row's end compute with the inputs of its last cell (so
+  // that they take the branches it takes) and do not store, since a wave of eight
+  // lanes or fewer issues about 3.5 times slower (65 x 64 x 64, chunks of 32 planes:
+  // a reinitialization stage 432 us, 120 us with all lanes).  FP32 waves of few
+  // lanes run as others do, and the lanes are left out.
+  const bool computes = sizeof(real_t) == 8 ? j <= a.fb.jhi : active;
+  const int ic = sizeof(real_t) == 8 ? min(i, a.fb.ihi) : i;
   // own column: needed by neighbours whenever it lies in the ghost box
   const bool own_in = i <= gb.ihi && j <= gb.jhi;
   const long long own = (long long)(i - gb.ilo) + (long long)a.sy * (j - gb.jlo);
@@ -151,9 +167,9 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
   const long long sz = a.sz;
 
   real_t ta0 = 0, tb0 = 0, ta1 = 0, tb1 = 0;
-  if (RHS == kAdvectDeform && active) {
-    ta0 = a.ta[0][i - gb.ilo];
-    tb0 = a.tb[0][i - gb.ilo];
+  if (RHS == kAdvectDeform && computes) {
+    ta0 = a.ta[0][ic - gb.ilo];
+    tb0 = a.tb[0][ic - gb.ilo];
     ta1 = a.ta[1][j - gb.jlo];
     tb1 = a.tb[1][j - gb.jlo];
   }
@@ -170,10 +186,10 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
   };
   auto load_in = [&](int k) {
     const long long zoff = sz * (k - gb.klo);
-    const long long off = own + zoff;
+    const long long off = own + zoff - (i - ic);
     In v{real_t(0), real_t(0), real_t(0), real_t(0), real_t(0)};
     if (hoff >= 0) v.hv = us[hoff + zoff];
-    if (active) {
+    if (computes) {
       if (STAGE != 1) v.uc = a.uc[off];
       if (RHS == kAdvectField) {
         v.c0 = a.vx[off];
@@ -195,46 +211,55 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
     plane[ly * PX + lx] = w[3];
     if (tid < NHALO) plane[hslot] = hv;
     __syncthreads();
-    if (active) {
-      real_t fx[7], fy[7], fz[7];
+    if (computes) {
+      const real_t* c = &plane[ly * PX + lx];
+      auto line = [&](real_t (&f)[7], int stride) {
 #pragma unroll
-      for (int s = -H; s <= H; s++) {
-        fx[s + 3] = plane[ly * PX + lx + s];
-        fy[s + 3] = plane[(ly + s) * PX + lx];
-        fz[s + 3] = w[s + 3];
-      }
-      real_t r;
+        for (int s = -H; s <= H; s++) f[s + 3] = c[s * stride];
+      };
+      real_t r, fx[7], fy[7];
+      line(fx, 1);
       if (sizeof(real_t) == 4 && RHS == kAdvectDeform) {
+        line(fy, PX);
         // r = -(u phi_x + v phi_y + w phi_z) with the derivatives' 1/dx folded into the velocity;
         // |u| < zero_tol  <=>  |u/dx| < zero_tol/dx
         const real_t ux = X0 * a.tb[2][k - gb.klo], vy = X1 * a.tb[2][k - gb.klo], wz = X2 * a.ta[2][k - gb.klo];
         const real_t px = fabs(ux) < kZeroTol * a.ix ? real_t(0) : weno_up(fx, real_t(1), ux > real_t(0));
         const real_t py = fabs(vy) < kZeroTol * a.iy ? real_t(0) : weno_up(fy, real_t(1), vy > real_t(0));
-        const real_t pz = fabs(wz) < kZeroTol * a.iz ? real_t(0) : weno_up(fz, real_t(1), wz > real_t(0));
+        const real_t pz = fabs(wz) < kZeroTol * a.iz ? real_t(0) : weno_up(w, real_t(1), wz > real_t(0));
         r = real_t(0) - (ux * px + vy * py + wz * pz);
       } else if (RHS == kAdvectField || RHS == kAdvectDeform) {
+        line(fy, PX);
         real_t u, v, vw;
         if (RHS == kAdvectField) {
           u = c0;
           v = c1;
           vw = c2;
         } else {
-          const real_t ta2 = a.ta[2][k - gb.klo], tb2 = a.tb[2][k - gb.klo], c = a.tfac;
-          u = real_t(2) * ta0 * tb1 * tb2 * c;
-          v = -(tb0 * ta1 * tb2 * c);
-          vw = -(tb0 * tb1 * ta2 * c);
+          const real_t ta2 = a.ta[2][k - gb.klo], tb2 = a.tb[2][k - gb.klo], tf = a.tfac;
+          u = real_t(2) * ta0 * tb1 * tb2 * tf;
+          v = -(tb0 * ta1 * tb2 * tf);
+          vw = -(tb0 * tb1 * ta2 * tf);
         }
         const real_t px = fabs(u) < kZeroTol ? real_t(0) : weno_up(fx, a.ix, u > real_t(0));
         const real_t py = fabs(v) < kZeroTol ? real_t(0) : weno_up(fy, a.iy, v > real_t(0));
-        const real_t pz = fabs(vw) < kZeroTol ? real_t(0) : weno_up(fz, a.iz, vw > real_t(0));
+        const real_t pz = fabs(vw) < kZeroTol ? real_t(0) : weno_up(w, a.iz, vw > real_t(0));
         r = real_t(0) - (u * px + v * py + vw * pz);
       } else {
+        // FP64 reads the line along y when x is done, and works on one axis at a
+        // time: the registers of two would cost a resident block
+        auto next_axis = [&](real_t& done) {
+          if (sizeof(real_t) == 8) asm volatile("" : "+v"(done) : : "memory");
+        };
         real_t xp, xm, yp, ym, zp, zm;
         weno_pm(fx, a.ix, xp, xm);
+        next_axis(xm);
+        line(fy, PX);
         weno_pm(fy, a.iy, yp, ym);
-        weno_pm(fz, a.iz, zp, zm);
+        next_axis(ym);
+        weno_pm(w, a.iz, zp, zm);
         if (RHS == kReinit) {
-          const real_t s = a.use_phi0 ? c0 : fx[3];
+          const real_t s = a.use_phi0 ? c0 : w[3];
           r = stage_reinit(s, a.use_phi0 != 0, xp, yp, zp, xm, ym, zm, a.dx_sq);
         } else {
           const real_t v = RHS == kNormalField ? c0 : a.vn;
@@ -242,8 +267,8 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
           if (fabs(v) >= kZeroTol) r = r - v * stage_sqrt(stencil::godunov_sq(v > real_t(0), xp, yp, zp, xm, ym, zm));
         }
       }
-      const real_t uc = STAGE == 1 ? fx[3] : ucv;
-      a.out[off] = rk_combine<STAGE>(uc, fx[3], a.dt, r);
+      const real_t uc = STAGE == 1 ? w[3] : ucv;
+      if (active) a.out[off] = rk_combine<STAGE>(uc, w[3], a.dt, r);
     }
   };
 

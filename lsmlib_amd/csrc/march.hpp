@@ -293,9 +293,14 @@ __global__ void __launch_bounds__(kMX* kMY) cross19_march_kernel(Box fb, View<co
 }
 
 // op.load(i, j, k) -> Op::In (pointwise inputs, issued before the plane's
-// barriers) and op.store(i, j, k, fx, fy, fz, in) at every cell of fb, where
-// f?[s + 3] = phi at offset s (|s| <= R) along x, y, z; phi must cover fb
-// widened by R cells on every side.  The plane with an R-cell x/y halo goes
+// barriers) and op.store(i, j, k, active, fx, fy, fz, in) on every row of the tile
+// inside fb, where f?[s + 3] = phi at offset s (|s| <= R) along x, y, z; phi must
+// cover fb widened by R cells on every side.  The lanes past the row's end load
+// the inputs of its last cell (so that they take the branches it takes) and store
+// with active false and lines of no meaning: an op computes for all lanes and
+// stores for the active ones, since an FP64 wave of eight lanes or fewer issues
+// about 3.5 times slower (the last tile of a row of 64 q + 1 .. 64 q + 8 cells:
+// 66 x 64 x 64, an upwinded WENO5 step 373 us, 203 us with all lanes).  The plane with an R-cell x/y halo goes
 // through LDS; the thread's own column from k - R to k + R is carried in
 // registers, with plane k + R + 1 in flight.
 template <int R, class Op>
@@ -337,7 +342,7 @@ __global__ void __launch_bounds__(kMX* kMY) line_march_kernel(Box fb, View<const
   for (int k = kb; k <= ke; k++) {
     const int dk = (k - kb) * sz;
     typename Op::In in{};
-    if (active) in = op.load(i, j, k);
+    if (j <= fb.jhi) in = op.load(min(i, fb.ihi), j, k);
     // the next cell's window and halo, needed only while k + 1 <= ke
     z[W] = own_in && k < ke ? phi.p[own + dk + (R + 1) * sz] : real_t(0);
     const real_t h1 = hoff >= 0 && k < ke ? phi.p[hoff + dk + sz] : real_t(0);
@@ -345,7 +350,7 @@ __global__ void __launch_bounds__(kMX* kMY) line_march_kernel(Box fb, View<const
     plane[slot] = z[R];
     if (tid < HALO) plane[hslot] = h0;
     __syncthreads();
-    if (active) {
+    if (j <= fb.jhi) {
       real_t fx[7] = {}, fy[7] = {}, fz[7] = {};
 #pragma unroll
       for (int s = -R; s <= R; s++) {
@@ -353,7 +358,7 @@ __global__ void __launch_bounds__(kMX* kMY) line_march_kernel(Box fb, View<const
         fy[s + 3] = plane[slot + s * PX];
         fz[s + 3] = z[s + R];
       }
-      op.store(i, j, k, fx, fy, fz, in);
+      op.store(i, j, k, active, fx, fy, fz, in);
     }
 #pragma unroll
     for (int s = 0; s < W; s++) z[s] = z[s + 1];

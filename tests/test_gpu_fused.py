@@ -184,3 +184,40 @@ def test_stage_does_not_depend_on_the_chunks(prec, n, kind):
         else:
             bound = 3 * 0.2 * 4 * 50 * 2.0 ** -24 * 2 * float(us.abs().max())
             assert float((a - b).abs().max()) <= bound, "stage %d" % stage
+
+
+# Rows whose last tile holds 1, 8 and 9 cells (the waves that compute for lanes past the row's end), and speeds that
+# change sign or vanish inside a wave (the waves that pick their side per lane).
+@pytest.mark.parametrize("nx", [1, 8, 65, 72, 73])
+@pytest.mark.parametrize("signs", ["minus", "plus", "mixed", "one lane", "zero"])
+def test_fp64_advection_by_lane_is_bitwise_the_oracle(nx, signs):
+    from lsmlib_amd.solver import Grid, Solver
+    g = Grid((nx, 5, 4), hi=(0.1 * nx, 0.45, 0.4))
+    s = Solver(g, "f64")
+    rng = np.random.default_rng(nx)
+    phi, phin = rng.standard_normal(g.shape), rng.standard_normal(g.shape)
+    vel = [np.abs(rng.standard_normal(g.shape)) + 0.1 for _ in range(3)]
+    if signs == "minus":
+        vel = [-v for v in vel]
+    elif signs == "mixed":
+        vel = [np.where(rng.random(g.shape) < 0.4, -v, np.where(rng.random(g.shape) < 0.1, 0.0, v)) for v in vel]
+    elif signs == "one lane":
+        for v in vel:
+            v[:, :, g.g + nx // 2] *= -1.0
+            v[:, :, g.g] = 1e-12
+    elif signs == "zero":
+        vel = [v * 1e-13 for v in vel]
+    ref = _oracle_stage(g, phi, phin, 2, 0.03, "advect", vel=vel)
+    out = s.field()
+    s.stage_advect(out, s.field(phi), s.field(phin), 2, 0.03, [s.field(v) for v in vel])
+    s.lib.check()
+    got = s.host(out)
+    assert np.array_equal(g.interior(got), g.interior(ref))
+    # the drop-in's upwinded derivatives on the same lanes
+    gb, fb, G = g.gb, g.fb, [s.field() for _ in range(4)]
+    o = [np.zeros(g.shape) for _ in range(4)]
+    s.lib.api.lsm3dupwindhjweno5(G[0], G[1], G[2], gb, s.field(phi), gb, *[s.field(v) for v in vel], gb, G[3], gb, fb,
+                                 *g.dx)
+    H.oracle().lsm3dupwindhjweno5(o[0], o[1], o[2], gb, phi, gb, *vel, gb, o[3], gb, fb, *g.dx)
+    for a, b in zip(G[:3], o[:3]):
+        assert np.array_equal(g.interior(s.host(a)), g.interior(b))
