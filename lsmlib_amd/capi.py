@@ -361,6 +361,31 @@ def _addr(x):
     raise TypeError("cannot take the address of %r" % type(x))
 
 
+# Pointers to the ints of a box or of an integer argument, by value: a time loop
+# passes the same few boxes at every call, and the C side only reads them.  Given
+# up whole when a program has used more than _MOST different ones.
+_MOST = 4096
+_BOXES: dict = {}
+_INTS: dict = {}
+
+
+def _box_pointers(box):
+    key = tuple(box)
+    ptrs = tuple(ctypes.byref(ctypes.c_int(int(v))) for v in key)
+    if len(_BOXES) >= _MOST:
+        _BOXES.clear()
+    _BOXES[key] = ptrs
+    return ptrs
+
+
+def _int_pointer(v):
+    ptr = ctypes.byref(ctypes.c_int(int(v)))
+    if len(_INTS) >= _MOST:
+        _INTS.clear()
+    _INTS[v] = ptr
+    return ptr
+
+
 class _Fn:
     def __init__(self, cfn, spec, real):
         self._f = cfn
@@ -370,47 +395,52 @@ class _Fn:
     def __call__(self, *args):
         if len(args) != len(self._spec):
             raise TypeError("expected %d arguments, got %d" % (len(self._spec), len(args)))
-        keep, cargs, outs = [], [], []
+        byref, c_void_p, real, boxes, ints = ctypes.byref, ctypes.c_void_p, self._real, _BOXES, _INTS
+        cargs, outs = [], []
+        add = cargs.append
         for (kind, name), a in zip(self._spec, args):
-            if kind in ("B", "Q"):
-                if len(a) != (6 if kind == "B" else 4):
-                    raise ValueError("box %s needs %d ints" % (name, 6 if kind == "B" else 4))
-                for v in a:
-                    c = ctypes.c_int(int(v))
-                    keep.append(c)
-                    cargs.append(ctypes.byref(c))
-            elif kind == "S":
-                c = self._real(float(a))
-                keep.append(c)
-                cargs.append(ctypes.byref(c))
-            elif kind == "SO":
-                c = self._real(0.0)
-                keep.append(c)
-                outs.append(c)
-                cargs.append(ctypes.byref(c))
-            elif kind == "I":
-                c = ctypes.c_int(int(a))
-                keep.append(c)
-                cargs.append(ctypes.byref(c))
-            elif kind == "IO":
-                c = ctypes.c_int(0 if a is None else int(a))
-                keep.append(c)
-                outs.append(c)
-                cargs.append(ctypes.byref(c))
-            elif kind == "U8":
-                c = ctypes.c_ubyte(int(a))
-                keep.append(c)
-                cargs.append(ctypes.byref(c))
-            else:  # R, IA, IH, M: addresses
-                ptr = _addr(a)
+            if kind == "R":
+                try:
+                    ptr = a.data_ptr()
+                except AttributeError:
+                    ptr = _addr(a)
                 if not ptr:  # every array of the table is required; a NULL one would be dereferenced
                     raise ValueError("array argument %s is NULL" % name)
-                cargs.append(ctypes.c_void_p(ptr))
+                add(c_void_p(ptr))
+            elif kind == "B" or kind == "Q":
+                if len(a) != (6 if kind == "B" else 4):
+                    raise ValueError("box %s needs %d ints" % (name, 6 if kind == "B" else 4))
+                try:
+                    ptrs = boxes[a]
+                except (KeyError, TypeError):  # a new box, or one that is no tuple
+                    ptrs = _box_pointers(a)
+                cargs += ptrs
+            elif kind == "S":
+                add(byref(real(a)))
+            elif kind == "I":
+                try:
+                    add(ints[a])
+                except (KeyError, TypeError):
+                    add(_int_pointer(a))
+            elif kind == "SO":
+                c = real(0.0)
+                outs.append(c)
+                add(byref(c))
+            elif kind == "IO":
+                c = ctypes.c_int(0 if a is None else int(a))
+                outs.append(c)
+                add(byref(c))
+            elif kind == "U8":
+                add(byref(ctypes.c_ubyte(int(a))))
+            else:  # IA, IH, M: addresses
+                ptr = _addr(a)
+                if not ptr:
+                    raise ValueError("array argument %s is NULL" % name)
+                add(c_void_p(ptr))
         self._f(*cargs)
-        vals = tuple(o.value for o in outs)
-        if not vals:
+        if not outs:
             return None
-        return vals[0] if len(vals) == 1 else vals
+        return outs[0].value if len(outs) == 1 else tuple(o.value for o in outs)
 
 
 class Bound:

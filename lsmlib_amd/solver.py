@@ -179,8 +179,9 @@ class Solver:
         self._velfill = L.fn("lsmhip_deform_velocity_fill", [P, P, P] + box + box + [P, R])
         self._vol = L.fn("lsmhip_volume_phi_lt0_f64",
                          [P, P] + box + box + [ctypes.POINTER(ctypes.c_double)] * 4)
-        self._gbp = [ctypes.c_int(v) for v in grid.gb]
-        self._fbp = [ctypes.c_int(v) for v in grid.fb]
+        # pointers to the boxes' ints, made once (the C side only reads them)
+        self._gbp = [ctypes.byref(ctypes.c_int(v)) for v in grid.gb]
+        self._fbp = [ctypes.byref(ctypes.c_int(v)) for v in grid.fb]
         self._tabs = None
 
     # -- memory ---------------------------------------------------------------
@@ -194,10 +195,10 @@ class Solver:
         return a.detach().to("cpu", self.torch.float64).numpy()
 
     def _gb(self):
-        return [ctypes.byref(v) for v in self._gbp]
+        return self._gbp
 
     def _fb(self):
-        return [ctypes.byref(v) for v in self._fbp]
+        return self._fbp
 
     def _ok(self, rc):
         if rc != 0:

@@ -2,11 +2,13 @@
 symbol include/*.h declares; the ctypes table covers the same drop-ins."""
 import ctypes
 import glob
+import math
 import os
 import re
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 from lsmlib_amd import capi
@@ -109,3 +111,19 @@ def test_prototypes_match_the_ctypes_table():
         assert len(got) == len(want), (sym, len(got), len(want))
         for pos, (g, w) in enumerate(zip(got, want)):
             assert g in w, (sym, pos, g, w)
+
+
+def test_binder_passes_each_call_its_own_values():
+    """Boxes and integer scalars go through pointers kept by value; more different ones than are kept, boxes given as
+    lists, and integers of other types reach the C side unchanged."""
+    seen = []
+    fn = capi._Fn(lambda *a: seen.append([getattr(x, "_obj", x).value for x in a]),
+                  [("R", "phi"), ("B", "gb"), ("Q", "fb"), ("I", "idx"), ("S", "dx"), ("U8", "mark")], ctypes.c_double)
+    phi = np.zeros(1)
+    for i in list(range(2 * capi._MOST)) + [0, 1]:
+        gb, fb = (-i, i, -1, 2, 3, i + 4), (0, i, -i, 5)
+        fn(phi, gb if i % 2 else list(gb), fb, np.int64(i) if i % 3 else i, -0.0 if i % 5 else 0.5 * i, i % 256)
+        got = seen.pop()
+        assert got == [phi.ctypes.data, *gb, *fb, i, -0.0 if i % 5 else 0.5 * i, i % 256]
+        assert math.copysign(1.0, got[12]) == (-1.0 if i % 5 else 1.0)
+    assert len(capi._BOXES) <= capi._MOST and len(capi._INTS) <= capi._MOST
