@@ -91,8 +91,8 @@ void face(const char* who, real_t* phi, const Box& gb, const Box& fb, int idx, i
 // with the face kernel's operations, and no ghost cell is read.
 //
 // The launch covers the ghost shell by lines normal to a face: one thread per
-// (i, j) column of the ghost box for the k ghost layers, one per (i, k) with
-// k interior for the j ghost layers, and eight lanes per (j, k) row with j and
+// (i, j) column of the ghost box and side for the k ghost layers, one per (i, k)
+// with k interior and side for the j ghost layers, and eight lanes per (j, k) row with j and
 // k interior for the i ghost layers (adjacent lanes write adjacent cells, so a
 // row's few ghost cells go out in one store request).  A line reads its edge
 // and next-inner values once and writes every ghost layer on that side from
@@ -109,59 +109,81 @@ __device__ __forceinline__ real_t extrap(real_t pb, real_t pin, int dist, int ki
   return pb + slope * real_t(dist);
 }
 
-// Value of cell (i, j, k) once the faces of axis 0 (v0: j, k interior) and of
-// axes 0..1 (v1: k interior) have been applied.
-__device__ __forceinline__ real_t shell_v0(const View<real_t>& P, const Shell& S, int i, int j, int k) {
-  const Box& f = S.fb;
-  if (i >= f.ilo && i <= f.ihi) return P(i, j, k);
-  const bool up = i > f.ihi;
-  if (S.kind == kPeriodic) return P(up ? i - f.nx() : i + f.nx(), j, k);
-  const int e = up ? f.ihi : f.ilo, n = up ? f.ihi - 1 : f.ilo + 1;
-  return extrap(P(e, j, k), S.kind == kCopy ? real_t(0) : P(n, j, k), up ? i - e : e - i, S.kind);
+// One index along an axis as the faces of that axis leave it: inside, or the
+// extrapolation (or periodic copy) of cells e and n; inside, e = n = the index.
+struct Along {
+  int e, n, dist;
+  bool in;
+};
+__device__ __forceinline__ Along along(int c, int lo, int hi, int kind) {
+  if (c >= lo && c <= hi) return Along{c, c, 0, true};
+  const bool up = c > hi;
+  if (kind == kPeriodic) {
+    const int w = up ? c - (hi - lo + 1) : c + (hi - lo + 1);
+    return Along{w, w, 0, true};  // the copy of one cell
+  }
+  const int e = up ? hi : lo;  // a copy takes e alone (n may lie outside a one-cell axis's box)
+  return Along{e, kind == kCopy ? e : up ? hi - 1 : lo + 1, up ? c - hi : lo - c, false};
 }
-__device__ __forceinline__ real_t shell_v1(const View<real_t>& P, const Shell& S, int i, int j, int k) {
-  const Box& f = S.fb;
-  if (j >= f.jlo && j <= f.jhi) return shell_v0(P, S, i, j, k);
-  const bool up = j > f.jhi;
-  if (S.kind == kPeriodic) return shell_v0(P, S, i, up ? j - f.ny() : j + f.ny(), k);
-  const int e = up ? f.jhi : f.jlo, n = up ? f.jhi - 1 : f.jlo + 1;
-  const real_t pb = shell_v0(P, S, i, e, k);
-  return extrap(pb, S.kind == kCopy ? real_t(0) : shell_v0(P, S, i, n, k), up ? j - e : e - j, S.kind);
+// From the values at e and n along one axis.
+__device__ __forceinline__ real_t face_value(const Along& a, real_t pe, real_t pn, int kind) {
+  return a.in ? pe : extrap(pe, pn, a.dist, kind);
+}
+// Value of cell (i, j, k) once the faces of axis 0 (v0: j, k interior) and of
+// axes 0..1 (v1: k interior) have been applied.  Every value that may enter is
+// loaded at once: behind a branch each would be a memory round trip of its own.
+__device__ __forceinline__ real_t shell_v0(const View<real_t>& P, int kind, const Along& x, int j, int k) {
+  const real_t pe = P(x.e, j, k), pn = P(x.n, j, k);
+  return face_value(x, pe, pn, kind);
+}
+__device__ __forceinline__ real_t shell_v1(const View<real_t>& P, int kind, const Along& x, const Along& y, int k) {
+  const real_t ee = P(x.e, y.e, k), ne = P(x.n, y.e, k), en = P(x.e, y.n, k), nn = P(x.n, y.n, k);
+  return face_value(y, face_value(x, ee, ne, kind), face_value(x, en, nn, kind), kind);
 }
 
+// The lines of the two sides of an axis go to different threads (the low side's
+// first): a line is one round of loads and its stores.  With both sides in one
+// thread and the corners' values behind branches, a fill waited for several
+// memory round trips in turn: signed linear FP32 at 64^3 7.5 -> 4.8 us, 203 x 149
+// x 97 7.3 -> 5.4, 256^3 9.4 -> 6.2, 512^3 17.5 both (bound by the strided lines).
 __global__ void __launch_bounds__(256) shell_kernel(View<real_t> P, Shell S) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const Box &g = S.gb, &f = S.fb;
-  if (t < S.lz) {  // column (i, j): the k ghost layers
-    const int nxg = g.nx(), c = (int)t;
+  if (t < 2 * S.lz) {  // column (i, j): the k ghost layers of one side
+    const bool up = t >= S.lz;
+    const int nxg = g.nx(), c = (int)(up ? t - S.lz : t);
     const int i = g.ilo + c % nxg, j = g.jlo + c / nxg;
-    for (int up = 0; up < 2; up++) {
-      const int k0 = up ? f.khi + 1 : g.klo, k1 = up ? g.khi : f.klo - 1;
-      if (S.kind == kPeriodic) {
-        for (int k = k0; k <= k1; k++) P(i, j, k) = shell_v1(P, S, i, j, up ? k - f.nz() : k + f.nz());
-      } else if (k0 <= k1) {
-        const int e = up ? f.khi : f.klo, n = up ? f.khi - 1 : f.klo + 1;
-        const real_t pb = shell_v1(P, S, i, j, e);
-        const real_t pin = S.kind == kCopy ? real_t(0) : shell_v1(P, S, i, j, n);
-        for (int k = k0; k <= k1; k++) P(i, j, k) = extrap(pb, pin, up ? k - e : e - k, S.kind);
+    const int k0 = up ? f.khi + 1 : g.klo, k1 = up ? g.khi : f.klo - 1;
+    const Along x = along(i, f.ilo, f.ihi, S.kind), y = along(j, f.jlo, f.jhi, S.kind);
+    if (S.kind == kPeriodic) {
+      for (int k = k0; k <= k1; k++) P(i, j, k) = P(x.e, y.e, up ? k - f.nz() : k + f.nz());
+    } else if (k0 <= k1) {
+      const int e = up ? f.khi : f.klo, n = S.kind == kCopy ? e : up ? f.khi - 1 : f.klo + 1;
+      real_t pb, pin;
+      if (__ballot(!(x.in && y.in)) != 0) {  // a wave with a column outside the fill box
+        pb = shell_v1(P, S.kind, x, y, e);
+        pin = shell_v1(P, S.kind, x, y, n);
+      } else {
+        pb = P(i, j, e);
+        pin = P(i, j, n);
       }
+      for (int k = k0; k <= k1; k++) P(i, j, k) = extrap(pb, pin, up ? k - e : e - k, S.kind);
     }
-  } else if (t < S.lz + S.ly) {  // row (i, k), k interior: the j ghost layers
-    const int nxg = g.nx(), c = (int)(t - S.lz);
+  } else if ((t -= 2 * S.lz) < 2 * S.ly) {  // row (i, k), k interior: the j ghost layers of one side
+    const bool up = t >= S.ly;
+    const int nxg = g.nx(), c = (int)(up ? t - S.ly : t);
     const int i = g.ilo + c % nxg, k = f.klo + c / nxg;
-    for (int up = 0; up < 2; up++) {
-      const int j0 = up ? f.jhi + 1 : g.jlo, j1 = up ? g.jhi : f.jlo - 1;
-      if (S.kind == kPeriodic) {
-        for (int j = j0; j <= j1; j++) P(i, j, k) = shell_v0(P, S, i, up ? j - f.ny() : j + f.ny(), k);
-      } else if (j0 <= j1) {
-        const int e = up ? f.jhi : f.jlo, n = up ? f.jhi - 1 : f.jlo + 1;
-        const real_t pb = shell_v0(P, S, i, e, k);
-        const real_t pin = S.kind == kCopy ? real_t(0) : shell_v0(P, S, i, n, k);
-        for (int j = j0; j <= j1; j++) P(i, j, k) = extrap(pb, pin, up ? j - e : e - j, S.kind);
-      }
+    const int j0 = up ? f.jhi + 1 : g.jlo, j1 = up ? g.jhi : f.jlo - 1;
+    const Along x = along(i, f.ilo, f.ihi, S.kind);
+    if (S.kind == kPeriodic) {
+      for (int j = j0; j <= j1; j++) P(i, j, k) = P(x.e, up ? j - f.ny() : j + f.ny(), k);
+    } else if (j0 <= j1) {
+      const int e = up ? f.jhi : f.jlo, n = S.kind == kCopy ? e : up ? f.jhi - 1 : f.jlo + 1;
+      const real_t pb = shell_v0(P, S.kind, x, e, k), pin = shell_v0(P, S.kind, x, n, k);
+      for (int j = j0; j <= j1; j++) P(i, j, k) = extrap(pb, pin, up ? j - e : e - j, S.kind);
     }
   } else {  // row (j, k), j and k interior: the i ghost layers, eight lanes per row
-    const long long u = t - S.lz - S.ly;
+    const long long u = t - 2 * S.ly;
     if (u >= 8 * S.lx) return;
     const int r = (int)(u >> 3), q = (int)(u & 7), nyi = f.ny();
     const int j = f.jlo + r % nyi, k = f.klo + r / nyi;
@@ -205,7 +227,7 @@ int shell(const char* who, real_t* phi, const Box& gb, const Box& fb, int kind) 
   S.lz = gz ? (long long)gb.nx() * gb.ny() : 0;
   S.ly = gy ? (long long)gb.nx() * fb.nz() : 0;
   S.lx = gx ? (long long)fb.ny() * fb.nz() : 0;
-  const long long threads = S.lz + S.ly + 8 * S.lx;
+  const long long threads = 2 * S.lz + 2 * S.ly + 8 * S.lx;
   if (threads == 0) return 0;
   hipLaunchKernelGGL(shell_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream(), view(phi, gb), S);
   return finish(who) ? 0 : -1;

@@ -232,6 +232,35 @@ def test_fill_all_faces_in_one_launch(kind, prec, boxes):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("kind,boxes", [
+    # one cell along x with ghosts on one side only, along z on both (a copy needs no second layer)
+    (2, ((-2, 0, -3, 4, -1, 2), (0, 0, 0, 3, 0, 0))),
+    (2, ((0, 3, 0, 2, -2, 0), (0, 3, 0, 0, 0, 0))),
+    # rows of several waves, with and without columns outside the fill box in a wave
+    *[(kind, ((-3, 200, -1, 8, -3, 6), (0, 197, 0, 6, 0, 4))) for kind in range(4)],
+    *[(kind, ((0, 130, 0, 70, -1, 5), (0, 130, 0, 70, 0, 4))) for kind in range(4)]])
+def test_fill_all_faces_by_wave(hip, kind, boxes):
+    """The one-launch fill against the oracle's faces in order, bit for bit, on guarded memory."""
+    import ctypes
+    import torch
+    gb, fb = boxes
+    rng = np.random.default_rng(kind)
+    phi = rng.standard_normal(H.shape_of(gb))
+    box = [ctypes.POINTER(ctypes.c_int)] * 6
+    fill = hip.fn("lsmhip_fill_ghosts", [ctypes.c_void_p] + box + box + [ctypes.c_int, ctypes.c_int])
+    bx = lambda b: [ctypes.byref(ctypes.c_int(v)) for v in b]  # noqa: E731
+    pad = 4096
+    buf = torch.full((phi.size + 2 * pad,), 7.5, dtype=torch.float64, device="cuda")
+    buf[pad:-pad] = torch.from_numpy(phi.reshape(-1)).cuda()
+    assert fill(buf.data_ptr() + 8 * pad, *bx(gb), *bx(fb), 9, kind) == 0
+    hip.check()
+    want = phi.copy()
+    for idx in range(6):
+        getattr(H.oracle(), FACE_SYM[kind])(want, gb, fb, idx)
+    assert np.array_equal(buf[pad:-pad].cpu().numpy().reshape(phi.shape), want)
+    assert (buf[:pad] == 7.5).all() and (buf[-pad:] == 7.5).all()
+
+
 @pytest.mark.parametrize("lo,hi", [(-160, -140), (-40, 28), (29, 31), (-160, 72), (70, 160)])
 def test_weno5_over_the_exponent_range(hip, lo, hi):
     """HJ-WENO5, plain and upwinded, bitwise where differences of a reconstruction span 10^lo .. 10^hi: the squares
