@@ -43,6 +43,7 @@ struct PlusMinusLine {
         plus.o[d](i, j, k) = p;
         minus.o[d](i, j, k) = m;
       }
+      if (ORDER == 5 && sizeof(real_t) == 8) asm volatile("" : "+v"(m) : : "memory");  // one axis at a time (registers)
     }
   }
 };

@@ -62,16 +62,8 @@ __device__ __forceinline__ void deform_velocity(const real_t* const ta[3], const
 
 // WENO5 derivatives of the fused stage: the reference's operation order in
 // FP64 (bitwise equal to the drop-in chain), the rearranged FP32 forms in FP32.
-// (stencil::plus_minus<5>, with the minus window's inputs tied to the plus
-// derivative: formed side by side the two windows need 140 registers and leave
-// one block to a CU instead of two)
 __device__ __forceinline__ void weno_pm(const double f[7], double inv, double& p, double& m) {
-  double v[6];
-#pragma unroll
-  for (int s = 0; s < 6; s++) v[s] = (f[s + 1] - f[s]) * inv;
-  p = stencil::weno5(v[5], v[4], v[3], v[2], v[1]);
-  asm volatile("" : "+v"(p), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]));
-  m = stencil::weno5(v[0], v[1], v[2], v[3], v[4]);
+  stencil::plus_minus<5>(f, inv, p, m);
 }
 __device__ __forceinline__ void weno_pm(const float f[7], float inv, float& p, float& m) {
   stencil::fastf::plus_minus(f, inv, p, m);

@@ -4,7 +4,7 @@
 // side along each axis (ENO / WENO, R <= 3).
 //
 // A block owns a kMX x kMY tile of the (i, j) plane and marches along k
-// through a chunk of kChunk planes.  Each thread keeps its own column at k-1,
+// through a chunk of planes (kChunk, fewer on small grids).  Each thread keeps its own column at k-1,
 // k, k+1 in registers and has the next plane's values (own column and halo) in
 // flight while the current plane is worked on; the current plane with a
 // one-cell x/y halo is staged in LDS,
@@ -29,9 +29,28 @@ struct Tiles {
   int nti, ntj, ntk, kc;
 };
 
-inline Tiles tiles_for(const Box& fb) {
-  return Tiles{(fb.nx() + kMX - 1) / kMX, (fb.ny() + kMY - 1) / kMY, (fb.nz() + kChunk - 1) / kChunk, kChunk};
+// Planes per chunk of tiles nti x ntj over nz planes: kChunk where that gives
+// 8192 blocks or more, else at most 8, and fewer where it would give less than
+// 1024 blocks (a block marches through its planes one after the other, so few
+// long chunks leave most of the chip idle), evened out over the planes.
+// Measured, chunks of 16 planes -> this rule, us: FP64 HJ-WENO5 64^3 57 -> 14,
+// 128^3 69 -> 63, 203 x 149 x 97 145 -> 106, 200^3 275 -> 246; FP32 HJ-WENO5 64^3
+// 24 -> 8, 128^3 28 -> 23; FP64 central gradient 64^3 12 -> 6, 200^3 82 -> 76; FP64
+// curvature 128^3 24 -> 21.  256^3 the same with 8, 12 and 16 planes.
+inline int chunk_planes(int nti, int ntj, int nz) {
+  const long long planes = (long long)nti * ntj * nz;
+  if (planes >= 8192LL * kChunk) return kChunk;
+  const long long fit = planes / 1024;
+  const int kc = fit < 1 ? 1 : fit > 8 ? 8 : (int)fit;
+  const int chunks = (nz + kc - 1) / kc;
+  return (nz + chunks - 1) / chunks;
 }
+inline Tiles tiles_of_width(const Box& fb, int width) {
+  const int nti = (fb.nx() + width - 1) / width, ntj = (fb.ny() + kMY - 1) / kMY;
+  const int kc = chunk_planes(nti, ntj, fb.nz());
+  return Tiles{nti, ntj, (fb.nz() + kc - 1) / kc, kc};
+}
+inline Tiles tiles_for(const Box& fb) { return tiles_of_width(fb, kMX); }
 inline dim3 grid_for(const Tiles& t) {
   const long long n = (long long)t.nti * t.ntj * t.ntk;
   return dim3((unsigned)(((n + 7) / 8) * 8));
@@ -117,9 +136,7 @@ __global__ void __launch_bounds__(kMX* kMY) star_march_kernel(Box fb, View<const
 // i0 + x and i0 + kMX + x of a 2 kMX x kMY tile.  Per cache-line request a
 // plane row then carries 512 rather than 256 bytes of FP32 (1024 / 512 of
 // FP64), and the two one-cell halo columns serve twice the cells.
-inline Tiles tiles_for_x2(const Box& fb) {
-  return Tiles{(fb.nx() + 2 * kMX - 1) / (2 * kMX), (fb.ny() + kMY - 1) / kMY, (fb.nz() + kChunk - 1) / kChunk, kChunk};
-}
+inline Tiles tiles_for_x2(const Box& fb) { return tiles_of_width(fb, 2 * kMX); }
 template <class Op>
 __global__ void __launch_bounds__(kMX* kMY) star_march_x2_kernel(Box fb, View<const real_t> phi, Tiles tl, Op op) {
   constexpr int TW = 2 * kMX, PX = TW + 2, PLANE = PX * (kMY + 2), HALO = PLANE - TW * kMY;

@@ -167,6 +167,10 @@ __device__ __forceinline__ void plus_minus(const T f[7], T inv, T& p, T& m) {
 #pragma unroll
     for (int s = -2; s <= 3; s++) v[s + 2] = LSM_D1(s) * inv;
     p = weno5(v[5], v[4], v[3], v[2], v[1]);
+    // FP64: the minus window waits for the plus derivative.  Formed side by side
+    // the two need up to 140 registers in the marching kernels, which leaves one
+    // or two blocks to a CU instead of three.
+    if constexpr (sizeof(T) == 8) asm volatile("" : "+v"(p), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]));
     m = weno5(v[0], v[1], v[2], v[3], v[4]);
   }
 }
