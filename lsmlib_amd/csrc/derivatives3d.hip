@@ -233,8 +233,7 @@ __global__ void __launch_bounds__(march::kMX* march::kMY)
   F h0 = hoff >= 0 ? phi.p[hoff] : F(0);
   // minus derivative along z at the first plane, from its window D(k-2 .. k+2)
   F zm, unused;
-  fwd_rev(win5(z[1] - z[0], z[2] - z[1], z[3] - z[2], z[4] - z[3], z[5] - z[4]), z[2] - z[1], z[3] - z[2],
-          z[4] - z[3], zm, unused);
+  fwd_rev(win5(z[1] - z[0], z[2] - z[1], z[3] - z[2], z[4] - z[3], z[5] - z[4]), z[3] - z[2], zm, unused);
   for (int k = kb; k <= ke; k++) {
     const int dk = (k - kb) * sz;
     z[7] = own_in && k < ke ? phi.p[own + dk + (R + 1) * sz] : F(0);
@@ -250,26 +249,25 @@ __global__ void __launch_bounds__(march::kMX* march::kMY)
       dy[q + 2] = plane[slot + q * PX] - plane[slot + (q - 1) * PX];
     }
     F xm, xpp, ym, ypp, zmn, zp;
-    fwd_rev(win5(dx[0], dx[1], dx[2], dx[3], dx[4]), dx[1], dx[2], dx[3], xm, xpp);
+    fwd_rev(win5(dx[0], dx[1], dx[2], dx[3], dx[4]), dx[2], xm, xpp);
     xplus[threadIdx.y][threadIdx.x] = xpp * ix;
     if (threadIdx.y == 0 && threadIdx.x < MY) {  // the column one past the tile, one row per lane
       const int row = ((int)threadIdx.x + R) * PX + MX + R;
       F e[5], ef, er;
 #pragma unroll
       for (int q = -2; q <= 2; q++) e[q + 2] = plane[row + q] - plane[row + q - 1];
-      fwd_rev(win5(e[0], e[1], e[2], e[3], e[4]), e[1], e[2], e[3], ef, er);
+      fwd_rev(win5(e[0], e[1], e[2], e[3], e[4]), e[2], ef, er);
       xplus[threadIdx.x][MX] = er * ix;
     }
-    fwd_rev(win5(dy[0], dy[1], dy[2], dy[3], dy[4]), dy[1], dy[2], dy[3], ym, ypp);
+    fwd_rev(win5(dy[0], dy[1], dy[2], dy[3], dy[4]), dy[2], ym, ypp);
     yplus[threadIdx.y][threadIdx.x] = ypp * iy;
     // z: the window D(k-1 .. k+3) gives the plus derivative here and the minus one at k + 1
-    fwd_rev(win5(z[2] - z[1], z[3] - z[2], z[4] - z[3], z[5] - z[4], z[6] - z[5]), z[3] - z[2], z[4] - z[3],
-            z[5] - z[4], zmn, zp);
+    fwd_rev(win5(z[2] - z[1], z[3] - z[2], z[4] - z[3], z[5] - z[4], z[6] - z[5]), z[4] - z[3], zmn, zp);
     __syncthreads();
     F yp;
     if (threadIdx.y == MY - 1) {  // the row past the tile
       F nf, nr;
-      fwd_rev(win5(dy[1], dy[2], dy[3], dy[4], dy[5]), dy[2], dy[3], dy[4], nf, nr);
+      fwd_rev(win5(dy[1], dy[2], dy[3], dy[4], dy[5]), dy[3], nf, nr);
       yp = nr * iy;
     } else {
       yp = yplus[threadIdx.y + 1][threadIdx.x];

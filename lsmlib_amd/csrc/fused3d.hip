@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
   for (int q = 0; q < 4; q++) dz[q] = zw[q + 2] - zw[q + 1];
   // minus derivative of the first plane, from its window D(k-2..k+2)
   F zm_next, zp_unused;
-  fwd_rev(win5(zw[1] - zw[0], dz[0], dz[1], dz[2], dz[3]), dz[0], dz[1], dz[2], zm_next, zp_unused);
+  fwd_rev(win5(zw[1] - zw[0], dz[0], dz[1], dz[2], dz[3]), dz[1], zm_next, zp_unused);
   zm_next *= iz;
 
   for (int k = kb; k <= ke; k++) {
@@ -385,7 +385,7 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
     dz[4] = zw[6] - zw[5];
     const Win wz1 = win5(dz[0], dz[1], dz[2], dz[3], dz[4]);
     float zpf, zmf;
-    fwd_rev(wz1, dz[1], dz[2], dz[3], zmf, zpf);
+    fwd_rev(wz1, dz[2], zmf, zpf);
     const float zp = zpf * iz;
     const float zm = zm_next;
     zm_next = zmf * iz;
@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
     }
     const Win wx = win5(dx_[0], dx_[1], dx_[2], dx_[3], dx_[4]);
     float xmf, xpf;
-    fwd_rev(wx, dx_[1], dx_[2], dx_[3], xmf, xpf);
+    fwd_rev(wx, dx_[2], xmf, xpf);
     const float xm = xmf * ix;
     xplus[threadIdx.y][threadIdx.x] = xpf * ix;
     if (threadIdx.y == 0 && threadIdx.x < TY) {  // one wave forms the TY plus derivatives of the tile's last column
@@ -408,20 +408,20 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
 #pragma unroll
       for (int q = -2; q <= 2; q++) e[q + 2] = plane[row + q] - plane[row + q - 1];
       float ef, er;
-      fwd_rev(win5(e[0], e[1], e[2], e[3], e[4]), e[1], e[2], e[3], ef, er);
+      fwd_rev(win5(e[0], e[1], e[2], e[3], e[4]), e[2], ef, er);
       xplus[threadIdx.x][TX] = er * ix;
     }
     // y: likewise along j
     const Win wy = win5(dy_[0], dy_[1], dy_[2], dy_[3], dy_[4]);
     float ymf, ypf;
-    fwd_rev(wy, dy_[1], dy_[2], dy_[3], ymf, ypf);
+    fwd_rev(wy, dy_[2], ymf, ypf);
     const float ym = ymf * iy;
     yplus[threadIdx.y][threadIdx.x] = ypf * iy;
     __syncthreads();
     float yp;
     if (threadIdx.y == TY - 1) {  // the last row forms the plus derivative from the row past the tile
       float nf, nr;
-      fwd_rev(win5(dy_[1], dy_[2], dy_[3], dy_[4], dy_[5]), dy_[2], dy_[3], dy_[4], nf, nr);
+      fwd_rev(win5(dy_[1], dy_[2], dy_[3], dy_[4], dy_[5]), dy_[3], nf, nr);
       yp = nr * iy;
     } else {
       yp = yplus[threadIdx.y + 1][threadIdx.x];
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
         const F v = RHS == kNormalField ? c0 : a.vn;
         r = 0.f;
         if (fabsf(v) >= kZeroTol)
-          r = r - v * __builtin_amdgcn_sqrtf(stencil::godunov_sq(v > 0.f, xp, yp, zp, xm, ym, zm));
+          r = r - v * __builtin_amdgcn_sqrtf(stencil::fastf::godunov_sq(v > 0.f, xp, yp, zp, xm, ym, zm));
       }
       const F uc = STAGE == 1 ? zw[3] : ucv;
       a.out[off] = rk_combine<STAGE>(uc, zw[3], a.dt, r);

@@ -104,10 +104,8 @@ __device__ __forceinline__ void plus_minus_local(const LocalStage& a, const real
     minus = stencil::weno5(dd[0] * inv, dd[1] * inv, dd[2] * inv, dd[3] * inv, dd[4] * inv);
   } else {
     using namespace stencil::fastf;
-    plus = (real_t)rev(win5((float)dd[1], (float)dd[2], (float)dd[3], (float)dd[4], (float)dd[5]), (float)dd[2],
-                       (float)dd[3], (float)dd[4]) * inv;
-    minus = (real_t)fwd(win5((float)dd[0], (float)dd[1], (float)dd[2], (float)dd[3], (float)dd[4]), (float)dd[1],
-                        (float)dd[2], (float)dd[3]) * inv;
+    plus = (real_t)rev(win5((float)dd[1], (float)dd[2], (float)dd[3], (float)dd[4], (float)dd[5]), (float)dd[3]) * inv;
+    minus = (real_t)fwd(win5((float)dd[0], (float)dd[1], (float)dd[2], (float)dd[3], (float)dd[4]), (float)dd[2]) * inv;
   }
 }
 

@@ -325,69 +325,74 @@ namespace fastf {
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // One WENO5 stencil (v1..v5) in two parts.  win5 holds what depends on the
-// five values as a set -- the normalised smoothness products and the
-// candidate differences; fwd finishes weno5(v1, .., v5) and rev finishes
-// weno5(v5, .., v1), whose smoothness indicators are those of the forward
-// order taken in reverse.  The plus derivative at a cell and the minus
-// derivative at the next cell along an axis use the same five differences in
-// opposite orders, so one window serves both.
+// five values as a set -- the normalised smoothness products, the candidate
+// differences and two of the differences t_ij = v_j - v_i; fwd finishes
+// weno5(v1, .., v5) and rev finishes weno5(v5, .., v1), whose smoothness
+// indicators are those of the forward order taken in reverse.  The plus
+// derivative at a cell and the minus derivative at the next cell along an axis
+// use the same five differences in opposite orders, so one window serves both.
 //
 // The nonlinear weights are unchanged when the smoothness indicators S_k and
 // eps = 1e-6 max v^2 are scaled together: win5 divides them by max v^2
-// ((max |v|)^2, exact as rounding is monotonic) and multiplies by 4, so that
-// 4 S_k = (13/3) a_k^2 + b_k^2 with a_k, b_k the reference's two terms.  With
-// alpha_k = d_k / e_k^2 over the common denominator e1^2 e2^2 e3^2 and
-// p1 - p2 = (a1 - a2)/3, p3 - p2 = (a2 - a3)/6,
-//   sum_k w_k p_k = p2 + (0.1 q23 (a1 - a2)/3 + 0.3 q12 (a2 - a3)/6) / sum_k d_k q_(other two).
+// ((max |v|)^2, exact as rounding is monotonic).  With a1 = t23 - t12,
+// a2 = t34 - t23, a3 = t45 - t34 the reference's
+// S_k = 13/12 (second difference)^2 + 1/4 (first difference)^2 are
+//   S1 = a1 (4/3 a1 + t23) + t23^2,  S3 = a3 (4/3 a3 - t34) + t34^2,
+//   S2 = 4/3 (t23^2 + t34^2 - 5/4 t23 t34),
+// each at least 0.8 of its largest square, so nothing cancels.  With alpha_k =
+// d_k / e_k^2 over the common denominator e1^2 e2^2 e3^2 and p1 - p2 = (a1 - a2)/3,
+// p3 - p2 = (a2 - a3)/6, p2 = v3 + t34/3 + t23/6,
+//   sum_k w_k p_k = p2 + (q23 (a1 - a2)/3 + q12 (a2 - a3)/2) / (q23 + 6 q13 + 3 q12).
+// 47 VALU instructions a derivative from its six values, 52 with S_k formed as
+// two squares each (advection cell-stage 181 -> @@, reinitialization 240 -> @@).
 struct Win {
-  float q12, q13, q23, d12, d23;
+  float q12, q13, q23, d12, d23, t23, t34;
 };
 
 __device__ __forceinline__ Win win5(float v1, float v2, float v3, float v4, float v5) {
   const float ma = fmaxf(fmaxf(fmaxf(fmaxf(fabsf(v1), fabsf(v2)), fabsf(v3)), fabsf(v4)), fabsf(v5));
   const float im = rcp(fmaf(ma, ma, 1e-30f));
-  const float a1 = fmaf(-2.f, v2, v1) + v3, b1 = fmaf(3.f, v3, fmaf(-4.f, v2, v1));
-  const float a2 = fmaf(-2.f, v3, v2) + v4, b2 = v2 - v4;
-  const float a3 = fmaf(-2.f, v4, v3) + v5, b3 = fmaf(3.f, v3, fmaf(-4.f, v4, v5));
-  const float e1 = fmaf(fmaf(a1 * (13.f / 3.f), a1, b1 * b1), im, 4e-6f);
-  const float e2 = fmaf(fmaf(a2 * (13.f / 3.f), a2, b2 * b2), im, 4e-6f);
-  const float e3 = fmaf(fmaf(a3 * (13.f / 3.f), a3, b3 * b3), im, 4e-6f);
+  const float t12 = v2 - v1, t23 = v3 - v2, t34 = v4 - v3, t45 = v5 - v4;
+  const float a1 = t23 - t12, a2 = t34 - t23, a3 = t45 - t34;
+  const float T2 = t23 * t23, T3 = t34 * t34;
+  const float e1 = fmaf(fmaf(a1, fmaf(4.f / 3.f, a1, t23), T2), im, 1e-6f);
+  const float e2 = fmaf(fmaf(-1.25f * t23, t34, T2 + T3), im * (4.f / 3.f), 1e-6f);
+  const float e3 = fmaf(fmaf(a3, fmaf(4.f / 3.f, a3, -t34), T3), im, 1e-6f);
   const float q1 = e1 * e1, q2 = e2 * e2, q3 = e3 * e3;
-  return Win{q1 * q2, q1 * q3, q2 * q3, a1 - a2, a2 - a3};
+  return Win{q1 * q2, q1 * q3, q2 * q3, a1 - a2, a2 - a3, t23, t34};
 }
 // weno5(v1, .., v5) from win5(v1, .., v5)
-__device__ __forceinline__ float fwd(const Win& w, float v2, float v3, float v4) {
-  const float den = fmaf(0.1f, w.q23, fmaf(0.6f, w.q13, 0.3f * w.q12));
-  const float num = fmaf(w.q23, w.d12 * (0.1f / 3.f), w.q12 * (w.d23 * 0.05f));
-  const float p2 = fmaf(-1.f / 6.f, v2, fmaf(5.f / 6.f, v3, (1.f / 3.f) * v4));
+__device__ __forceinline__ float fwd(const Win& w, float v3) {
+  const float den = fmaf(6.f, w.q13, fmaf(3.f, w.q12, w.q23));
+  const float num = fmaf(w.q23, w.d12 * (1.f / 3.f), w.q12 * (w.d23 * 0.5f));
+  const float p2 = fmaf(1.f / 3.f, w.t34, fmaf(1.f / 6.f, w.t23, v3));
   return fmaf(num, rcp(den), p2);
 }
-// weno5(v5, .., v1) from win5(v1, .., v5): S1 and S3 trade places, and the
-// candidate differences become -(a2 - a3) and -(a1 - a2)
-__device__ __forceinline__ float rev(const Win& w, float v2, float v3, float v4) {
-  const float den = fmaf(0.1f, w.q12, fmaf(0.6f, w.q13, 0.3f * w.q23));
-  const float num = -fmaf(w.q12, w.d23 * (0.1f / 3.f), w.q23 * (w.d12 * 0.05f));
-  const float p2 = fmaf(-1.f / 6.f, v4, fmaf(5.f / 6.f, v3, (1.f / 3.f) * v2));
+// weno5(v5, .., v1) from win5(v1, .., v5): S1 and S3 trade places, the
+// candidate differences become -(a2 - a3) and -(a1 - a2), t23 and t34 become
+// -t34 and -t23
+__device__ __forceinline__ float rev(const Win& w, float v3) {
+  const float den = fmaf(6.f, w.q13, fmaf(3.f, w.q23, w.q12));
+  const float num = -fmaf(w.q12, w.d23 * (1.f / 3.f), w.q23 * (w.d12 * 0.5f));
+  const float p2 = fmaf(-1.f / 3.f, w.t23, fmaf(-1.f / 6.f, w.t34, v3));
   return fmaf(num, rcp(den), p2);
 }
 
 __device__ __forceinline__ float weno5(float v1, float v2, float v3, float v4, float v5) {
-  return fwd(win5(v1, v2, v3, v4, v5), v2, v3, v4);
+  return fwd(win5(v1, v2, v3, v4, v5), v3);
 }
 // fwd and rev of one window together (the minus derivative at a cell and the
-// plus derivative at the cell before it): the two denominators share 0.6 q13,
-// the numerators the products q23 d12 and q12 d23, the linear parts (5/6) v3.
-// The same weights and candidates as fwd and rev, rounded in another order.
-__device__ __forceinline__ void fwd_rev(const Win& w, float v2, float v3, float v4, float& f, float& r) {
-  const float m13 = 0.6f * w.q13;
-  const float den_f = fmaf(0.1f, w.q23, fmaf(0.3f, w.q12, m13));
-  const float den_r = fmaf(0.1f, w.q12, fmaf(0.3f, w.q23, m13));
+// plus derivative at the cell before it), the numerators sharing the products
+// q23 d12 and q12 d23.  The same weights and candidates as fwd and rev, rounded
+// in another order.
+__device__ __forceinline__ void fwd_rev(const Win& w, float v3, float& f, float& r) {
+  const float den_f = fmaf(6.f, w.q13, fmaf(3.f, w.q12, w.q23));
+  const float den_r = fmaf(6.f, w.q13, fmaf(3.f, w.q23, w.q12));
   const float pa = w.q23 * w.d12, pb = w.q12 * w.d23;
-  const float num_f = fmaf(0.1f / 3.f, pa, 0.05f * pb);
-  const float num_r = -fmaf(0.1f / 3.f, pb, 0.05f * pa);
-  const float t3 = (5.f / 6.f) * v3;
-  const float p2_f = fmaf(-1.f / 6.f, v2, fmaf(1.f / 3.f, v4, t3));
-  const float p2_r = fmaf(-1.f / 6.f, v4, fmaf(1.f / 3.f, v2, t3));
+  const float num_f = fmaf(1.f / 3.f, pa, 0.5f * pb);
+  const float num_r = -fmaf(1.f / 3.f, pb, 0.5f * pa);
+  const float p2_f = fmaf(1.f / 3.f, w.t34, fmaf(1.f / 6.f, w.t23, v3));
+  const float p2_r = fmaf(-1.f / 3.f, w.t23, fmaf(-1.f / 6.f, w.t34, v3));
   f = fmaf(num_f, rcp(den_f), p2_f);
   r = fmaf(num_r, rcp(den_r), p2_r);
 }
@@ -398,8 +403,8 @@ __device__ __forceinline__ void plus_minus(const float f[7], float inv, float& p
   float d[6];
 #pragma unroll
   for (int s = -2; s <= 3; s++) d[s + 2] = f[s + 3] - f[s + 2];
-  p = rev(win5(d[1], d[2], d[3], d[4], d[5]), d[2], d[3], d[4]) * inv;
-  m = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[1], d[2], d[3]) * inv;
+  p = rev(win5(d[1], d[2], d[3], d[4], d[5]), d[3]) * inv;
+  m = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[2]) * inv;
 }
 
 // Velocity-upwinded WENO5 derivative (vpos: backward/minus stencil).
@@ -425,15 +430,32 @@ __device__ __forceinline__ float upwind_wave(const float f[7], float inv, bool v
   // tails would need register moves on every path)
   float r;
   if (pos == live) {
-    r = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[1], d[2], d[3]) * inv;
+    r = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[2]) * inv;
     asm volatile("" : "+v"(r));
   } else if (pos == 0) {
-    r = fwd(win5(d[5], d[4], d[3], d[2], d[1]), d[4], d[3], d[2]) * inv;
+    r = fwd(win5(d[5], d[4], d[3], d[2], d[1]), d[3]) * inv;
     asm volatile("" : "+v"(r));
   } else {
     r = upwind(f, inv, vpos);
   }
   return r;
+}
+
+// Godunov |grad phi|^2 for a front that moves outward (pos) or inward, or for the
+// reinitialization on the side of sign pos: per axis the square of
+// max(m, -p, 0), or of max(-m, p, 0).  The signs are flipped by an exclusive or
+// and the larger is squared once (the squares' maximum is the maximum's square).
+__device__ __forceinline__ float godunov_sq(bool pos, float xp, float yp, float zp, float xm, float ym, float zm) {
+  const unsigned fm = pos ? 0u : 0x80000000u, fp = fm ^ 0x80000000u;
+  const float gp[3] = {xp, yp, zp}, gm[3] = {xm, ym, zm};
+  float n2 = 0.f;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const float m = __uint_as_float(__float_as_uint(gm[d]) ^ fm), p = __uint_as_float(__float_as_uint(gp[d]) ^ fp);
+    const float st = fmaxf(fmaxf(m, p), 0.f);
+    n2 = fmaf(st, st, n2);
+  }
+  return n2;
 }
 
 // Reinitialization RHS of one cell (the reference's formula,
@@ -442,15 +464,7 @@ __device__ __forceinline__ float upwind_wave(const float f[7], float inv, bool v
 // rounded FP32 sqrt and division sequences.
 __device__ __forceinline__ float reinit_rhs(float s, bool use_phi0, float xp, float yp, float zp, float xm, float ym,
                                             float zm, float dx_sq) {
-  const float gp[3] = {xp, yp, zp}, gm[3] = {xm, ym, zm};
-  float n2 = 0.f;
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    const float p = s > 0.f ? fmaxf(-gp[d], 0.f) : fmaxf(gp[d], 0.f);
-    const float m = s > 0.f ? fmaxf(gm[d], 0.f) : fmaxf(-gm[d], 0.f);
-    const float st = fmaxf(p, m);
-    n2 = fmaf(st, st, n2);
-  }
+  const float n2 = godunov_sq(s > 0.f, xp, yp, zp, xm, ym, zm);
   if (!(fabsf(s) >= kZeroTol)) return 0.f;
   const float sgn = s * __builtin_amdgcn_rsqf(fmaf(s, s, use_phi0 ? dx_sq : n2 * dx_sq));
   return sgn * (1.f - __builtin_amdgcn_sqrtf(n2));
