@@ -69,11 +69,12 @@ __device__ __forceinline__ void weno_pm(const float f[7], float inv, float& p, f
   stencil::fastf::plus_minus(f, inv, p, m);
 }
 
-__device__ __forceinline__ double weno_up(const double f[7], double inv, bool vpos) {
-  return stencil::upwind<5>(f, inv, vpos);
+// (upwinded, 0 where |vel| < tol)
+__device__ __forceinline__ double weno_up(const double f[7], double inv, double vel, double tol) {
+  return fabs(vel) < tol ? 0.0 : stencil::upwind<5>(f, inv, vel > 0.0);
 }
-__device__ __forceinline__ float weno_up(const float f[7], float inv, bool vpos) {
-  return stencil::fastf::upwind_wave(f, inv, vpos);
+__device__ __forceinline__ float weno_up(const float f[7], float inv, float vel, float tol) {
+  return stencil::fastf::upwind_wave(f, inv, vel, tol);
 }
 
 // Square root and reinitialization RHS of the fused stages: the reference's
@@ -86,7 +87,28 @@ __device__ __forceinline__ double stage_reinit(double s, bool u0, double xp, dou
 }
 __device__ __forceinline__ float stage_reinit(float s, bool u0, float xp, float yp, float zp, float xm, float ym,
                                               float zm, float dx_sq) {
-  return stencil::fastf::reinit_rhs(s, u0, xp, yp, zp, xm, ym, zm, dx_sq);
+  return stencil::fastf::reinit_rhs(s, u0, stencil::fastf::godunov_sq(s > 0.f, xp, yp, zp, xm, ym, zm), dx_sq);
+}
+
+// Element of a plane: base is uniform (the plane's start), byte a lane's offset in
+// the plane.  A plane of an array below 2^31 elements with three ghost layers at
+// either end along k is below 2^32 bytes, so the address is a scalar base and a
+// 32-bit lane offset, with no 64-bit addition per access on the VALU.  (The asm
+// keeps the compiler from forming base + byte ahead of the march and adding to
+// that.)
+__device__ __forceinline__ real_t in_plane(const real_t* base, unsigned byte) {
+  asm volatile("" : "+v"(byte));
+  return *reinterpret_cast<const real_t*>(reinterpret_cast<const char*>(base) + byte);
+}
+__device__ __forceinline__ void to_plane(real_t* base, unsigned byte, real_t v) {
+  asm volatile("" : "+v"(byte));
+  *reinterpret_cast<real_t*>(reinterpret_cast<char*>(base) + byte) = v;
+}
+// Value of a table at a uniform index, through the scalar cache (the tables are
+// not written while a stage runs).
+__device__ __forceinline__ real_t uniform_value(const real_t* tab, int at) {
+  typedef const __attribute__((address_space(4))) real_t* table_t;
+  return ((table_t)tab)[at];
 }
 
 template <int STAGE>
@@ -116,7 +138,7 @@ __device__ __forceinline__ void halo_pos(int h, int& px, int& py) {
 }
 
 template <int RHS, int STAGE>
-__global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_stage_kernel(FusedArgs a) {
+__global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 8) fused_stage_kernel(FusedArgs a) {
   __shared__ real_t plane[PLANE];
   const int tid = threadIdx.y * TX + threadIdx.x;
 
@@ -142,17 +164,19 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
   const int ic = sizeof(real_t) == 8 ? min(i, a.fb.ihi) : i;
   // own column: needed by neighbours whenever it lies in the ghost box
   const bool own_in = i <= gb.ihi && j <= gb.jhi;
-  const long long own = (long long)(i - gb.ilo) + (long long)a.sy * (j - gb.jlo);
-  // halo element of this thread (the same slot in every plane), -1 when none or outside the ghost box
-  long long hoff = -1;
+  const unsigned own = (unsigned)((i - gb.ilo) + a.sy * (j - gb.jlo)) * (unsigned)sizeof(real_t);
+  const unsigned cell_in = own - (unsigned)(i - ic) * (unsigned)sizeof(real_t);  // the per-cell inputs' offset
+  // halo element of this thread (the same slot in every plane), unless it has none or it lies outside the ghost box
+  bool has_halo = false;
+  unsigned hoff = 0;
   int hslot = 0;
   if (tid < NHALO) {
     int px, py;
     halo_pos(tid, px, py);
     const int gi = i0 - H + px, gj = j0 - H + py;
     hslot = py * PX + px;
-    if (gi >= gb.ilo && gi <= gb.ihi && gj >= gb.jlo && gj <= gb.jhi)
-      hoff = (long long)(gi - gb.ilo) + (long long)a.sy * (gj - gb.jlo);
+    has_halo = gi >= gb.ilo && gi <= gb.ihi && gj >= gb.jlo && gj <= gb.jhi;
+    if (has_halo) hoff = (unsigned)((gi - gb.ilo) + a.sy * (gj - gb.jlo)) * (unsigned)sizeof(real_t);
   }
   const int lx = threadIdx.x + H, ly = threadIdx.y + H;
   const real_t* us = a.us;
@@ -171,34 +195,32 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
                X2 = -(a.tfac * a.iz) * tb0 * tb1;
 
   // plane k + d of the own column
-  auto zload = [&](int k, int d) { return own_in ? us[own + sz * (k + d - gb.klo)] : real_t(0); };
+  auto zload = [&](int k, int d) { return own_in ? in_plane(us + sz * (k + d - gb.klo), own) : real_t(0); };
   // the halo element and the per-cell inputs of plane k
   struct In {
     real_t hv, uc, c0, c1, c2;
   };
   auto load_in = [&](int k) {
     const long long zoff = sz * (k - gb.klo);
-    const long long off = own + zoff - (i - ic);
     In v{real_t(0), real_t(0), real_t(0), real_t(0), real_t(0)};
-    if (hoff >= 0) v.hv = us[hoff + zoff];
+    if (has_halo) v.hv = in_plane(us + zoff, hoff);
     if (computes) {
-      if (STAGE != 1) v.uc = a.uc[off];
+      if (STAGE != 1) v.uc = in_plane(a.uc + zoff, cell_in);
       if (RHS == kAdvectField) {
-        v.c0 = a.vx[off];
-        v.c1 = a.vy[off];
-        v.c2 = a.vz[off];
+        v.c0 = in_plane(a.vx + zoff, cell_in);
+        v.c1 = in_plane(a.vy + zoff, cell_in);
+        v.c2 = in_plane(a.vz + zoff, cell_in);
       } else if (RHS == kReinit) {
-        v.c0 = a.use_phi0 ? a.phi0[off] : real_t(0);
+        v.c0 = a.use_phi0 ? in_plane(a.phi0 + zoff, cell_in) : real_t(0);
       } else if (RHS == kNormalField) {
-        v.c0 = a.vnf[off];
+        v.c0 = in_plane(a.vnf + zoff, cell_in);
       }
     }
     return v;
   };
   // cell (i, j, k) with its z window w[s + 3] = u(i, j, k + s) and inputs in
   auto cell = [&](int k, const real_t (&w)[7], const In& in) {
-    const long long off = own + sz * (k - gb.klo);
-    const real_t hv = in.hv, ucv = in.uc, c0 = in.c0, c1 = in.c1, c2 = in.c2;
+    const real_t hv = in.hv, c0 = in.c0, c1 = in.c1, c2 = in.c2;
     __syncthreads();  // the previous plane's reads are done
     plane[ly * PX + lx] = w[3];
     if (tid < NHALO) plane[hslot] = hv;
@@ -215,10 +237,11 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
         line(fy, PX);
         // r = -(u phi_x + v phi_y + w phi_z) with the derivatives' 1/dx folded into the velocity;
         // |u| < zero_tol  <=>  |u/dx| < zero_tol/dx
-        const real_t ux = X0 * a.tb[2][k - gb.klo], vy = X1 * a.tb[2][k - gb.klo], wz = X2 * a.ta[2][k - gb.klo];
-        const real_t px = fabs(ux) < kZeroTol * a.ix ? real_t(0) : weno_up(fx, real_t(1), ux > real_t(0));
-        const real_t py = fabs(vy) < kZeroTol * a.iy ? real_t(0) : weno_up(fy, real_t(1), vy > real_t(0));
-        const real_t pz = fabs(wz) < kZeroTol * a.iz ? real_t(0) : weno_up(w, real_t(1), wz > real_t(0));
+        const real_t ta2 = uniform_value(a.ta[2], k - gb.klo), tb2 = uniform_value(a.tb[2], k - gb.klo);
+        const real_t ux = X0 * tb2, vy = X1 * tb2, wz = X2 * ta2;
+        const real_t px = weno_up(fx, real_t(1), ux, kZeroTol * a.ix);
+        const real_t py = weno_up(fy, real_t(1), vy, kZeroTol * a.iy);
+        const real_t pz = weno_up(w, real_t(1), wz, kZeroTol * a.iz);
         r = real_t(0) - (ux * px + vy * py + wz * pz);
       } else if (RHS == kAdvectField || RHS == kAdvectDeform) {
         line(fy, PX);
@@ -228,14 +251,14 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
           v = c1;
           vw = c2;
         } else {
-          const real_t ta2 = a.ta[2][k - gb.klo], tb2 = a.tb[2][k - gb.klo], tf = a.tfac;
+          const real_t ta2 = uniform_value(a.ta[2], k - gb.klo), tb2 = uniform_value(a.tb[2], k - gb.klo), tf = a.tfac;
           u = real_t(2) * ta0 * tb1 * tb2 * tf;
           v = -(tb0 * ta1 * tb2 * tf);
           vw = -(tb0 * tb1 * ta2 * tf);
         }
-        const real_t px = fabs(u) < kZeroTol ? real_t(0) : weno_up(fx, a.ix, u > real_t(0));
-        const real_t py = fabs(v) < kZeroTol ? real_t(0) : weno_up(fy, a.iy, v > real_t(0));
-        const real_t pz = fabs(vw) < kZeroTol ? real_t(0) : weno_up(w, a.iz, vw > real_t(0));
+        const real_t px = weno_up(fx, a.ix, u, kZeroTol);
+        const real_t py = weno_up(fy, a.iy, v, kZeroTol);
+        const real_t pz = weno_up(w, a.iz, vw, kZeroTol);
         r = real_t(0) - (u * px + v * py + vw * pz);
       } else {
         // FP64 reads the line along y when x is done, and works on one axis at a
@@ -259,8 +282,11 @@ __global__ void __launch_bounds__(TX* TY, sizeof(real_t) == 8 ? 4 : 1) fused_sta
           if (fabs(v) >= kZeroTol) r = r - v * stage_sqrt(stencil::godunov_sq(v > real_t(0), xp, yp, zp, xm, ym, zm));
         }
       }
-      const real_t uc = STAGE == 1 ? w[3] : ucv;
-      if (active) a.out[off] = rk_combine<STAGE>(uc, w[3], a.dt, r);
+      real_t uc = STAGE == 1 ? w[3] : in.uc;
+      // (the combination's product with uc stays here; formed where uc is loaded, a
+      // plane ahead, it would wait for the memory there)
+      asm volatile("" : "+v"(uc));
+      if (active) to_plane(a.out + sz * (k - gb.klo), own, rk_combine<STAGE>(uc, w[3], a.dt, r));
     }
   };
 
@@ -338,70 +364,72 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
   const Box gb = a.gb;
   const bool active = i <= a.fb.ihi && j <= a.fb.jhi;
   const bool own_in = i <= gb.ihi && j <= gb.jhi;
-  const long long own = (long long)(i - gb.ilo) + (long long)a.sy * (j - gb.jlo);
-  long long hoff = -1;
+  const unsigned own = (unsigned)((i - gb.ilo) + a.sy * (j - gb.jlo)) * (unsigned)sizeof(F);
+  bool has_halo = false;
+  unsigned hoff = 0;
   int hslot = 0;
   if (tid < NHALO) {
     int px, py;
     halo_pos(tid, px, py);
     const int gi = i0 - H + px, gj = j0 - H + py;
     hslot = py * PX + px;
-    if (gi >= gb.ilo && gi <= gb.ihi && gj >= gb.jlo && gj <= gb.jhi)
-      hoff = (long long)(gi - gb.ilo) + (long long)a.sy * (gj - gb.jlo);
+    has_halo = gi >= gb.ilo && gi <= gb.ihi && gj >= gb.jlo && gj <= gb.jhi;
+    if (has_halo) hoff = (unsigned)((gi - gb.ilo) + a.sy * (gj - gb.jlo)) * (unsigned)sizeof(F);
   }
   const int lx = threadIdx.x + H, ly = threadIdx.y + H;
   const F* us = a.us;
   const long long sz = a.sz;
-  const F ix = a.ix, iy = a.iy, iz = a.iz;
 
-  F zw[7];  // zw[s+3] = u(i, j, k+s)
-#pragma unroll
-  for (int s = 0; s < 6; s++) zw[s] = own_in ? us[own + sz * (kb - H + s - gb.klo)] : F(0);
-  F dz[5];  // dz[t] = D(k-1+t), D(m) = u(m) - u(m-1) along z
-#pragma unroll
-  for (int q = 0; q < 4; q++) dz[q] = zw[q + 2] - zw[q + 1];
-  // minus derivative of the first plane, from its window D(k-2..k+2)
+  // zw[s] = u(i, j, k+s), dz[t] = D(k-1+t), D(m) = u(m) - u(m-1) along z; the
+  // derivatives are in undivided units until one of an axis's two is taken
+  F zw[4], dz[5];
   F zm_next, zp_unused;
-  fwd_rev(win5(zw[1] - zw[0], dz[0], dz[1], dz[2], dz[3]), dz[1], zm_next, zp_unused);
-  zm_next *= iz;
+  {
+    F w[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) w[s] = own_in ? in_plane(us + sz * (kb - H + s - gb.klo), own) : F(0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) dz[q] = w[q + 2] - w[q + 1];
+#pragma unroll
+    for (int s = 0; s < 3; s++) zw[s] = w[s + 3];
+    // minus derivative of the first plane, from its window D(k-2..k+2)
+    fwd_rev(win5(w[1] - w[0], dz[0], dz[1], dz[2], dz[3]), dz[1], zm_next, zp_unused);
+  }
 
-  for (int k = kb; k <= ke; k++) {
+  F znew = F(0), hv = F(0), ucv = F(0), c0 = F(0);
+  auto step = [&](int k) {
     const long long zoff = sz * (k - gb.klo);
-    zw[6] = own_in ? us[own + zoff + H * sz] : F(0);
-    const F hv = hoff >= 0 ? us[hoff + zoff] : F(0);
-    const long long off = own + zoff;
-    const F ucv = STAGE != 1 && active ? a.uc[off] : F(0);
-    F c0 = F(0);
+    // (a lane outside keeps the zero it began with)
+    if (own_in) znew = in_plane(us + zoff + H * sz, own);
+    if (has_halo) hv = in_plane(us + zoff, hoff);
     if (active) {
-      if (RHS == kReinit) c0 = a.use_phi0 ? a.phi0[off] : F(0);
-      else if (RHS == kNormalField) c0 = a.vnf[off];
+      if (STAGE != 1) ucv = in_plane(a.uc + zoff, own);
+      if (RHS == kReinit && a.use_phi0) c0 = in_plane(a.phi0 + zoff, own);
+      else if (RHS == kNormalField) c0 = in_plane(a.vnf + zoff, own);
     }
+    zw[3] = znew;
     __syncthreads();
-    plane[ly * PX + lx] = zw[3];
+    plane[ly * PX + lx] = zw[0];
     if (tid < NHALO) plane[hslot] = hv;
     __syncthreads();
     // z: the window D(k-1..k+3) gives plus(k) and minus(k+1); minus(k) was
     // formed from the previous plane's window
-    dz[4] = zw[6] - zw[5];
-    const Win wz1 = win5(dz[0], dz[1], dz[2], dz[3], dz[4]);
-    float zpf, zmf;
-    fwd_rev(wz1, dz[2], zmf, zpf);
-    const float zp = zpf * iz;
+    dz[4] = zw[3] - zw[2];
+    float zp, zmf;
+    fwd_rev(win5(dz[0], dz[1], dz[2], dz[3], dz[4]), dz[2], zmf, zp);
     const float zm = zm_next;
-    zm_next = zmf * iz;
+    zm_next = zmf;
     // x: this cell's window D(i-2..i+2) gives its minus derivative and the plus
     // derivative of the cell before it
-    F dx_[6], dy_[6];
+    F dx_[5], dy_[6];
 #pragma unroll
     for (int q = -2; q <= 3; q++) {
-      dx_[q + 2] = plane[ly * PX + lx + q] - plane[ly * PX + lx + q - 1];
+      if (q < 3) dx_[q + 2] = plane[ly * PX + lx + q] - plane[ly * PX + lx + q - 1];
       dy_[q + 2] = plane[(ly + q) * PX + lx] - plane[(ly + q - 1) * PX + lx];
     }
-    const Win wx = win5(dx_[0], dx_[1], dx_[2], dx_[3], dx_[4]);
-    float xmf, xpf;
-    fwd_rev(wx, dx_[2], xmf, xpf);
-    const float xm = xmf * ix;
-    xplus[threadIdx.y][threadIdx.x] = xpf * ix;
+    float xm, xpf;
+    fwd_rev(win5(dx_[0], dx_[1], dx_[2], dx_[3], dx_[4]), dx_[2], xm, xpf);
+    xplus[threadIdx.y][threadIdx.x] = xpf;
     if (threadIdx.y == 0 && threadIdx.x < TY) {  // one wave forms the TY plus derivatives of the tile's last column
       const int row = (threadIdx.x + H) * PX + TX + H;
       F e[5];
@@ -409,20 +437,17 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
       for (int q = -2; q <= 2; q++) e[q + 2] = plane[row + q] - plane[row + q - 1];
       float ef, er;
       fwd_rev(win5(e[0], e[1], e[2], e[3], e[4]), e[2], ef, er);
-      xplus[threadIdx.x][TX] = er * ix;
+      xplus[threadIdx.x][TX] = er;
     }
     // y: likewise along j
-    const Win wy = win5(dy_[0], dy_[1], dy_[2], dy_[3], dy_[4]);
-    float ymf, ypf;
-    fwd_rev(wy, dy_[2], ymf, ypf);
-    const float ym = ymf * iy;
-    yplus[threadIdx.y][threadIdx.x] = ypf * iy;
+    float ym, ypf;
+    fwd_rev(win5(dy_[0], dy_[1], dy_[2], dy_[3], dy_[4]), dy_[2], ym, ypf);
+    yplus[threadIdx.y][threadIdx.x] = ypf;
     __syncthreads();
     float yp;
     if (threadIdx.y == TY - 1) {  // the last row forms the plus derivative from the row past the tile
-      float nf, nr;
-      fwd_rev(win5(dy_[1], dy_[2], dy_[3], dy_[4], dy_[5]), dy_[3], nf, nr);
-      yp = nr * iy;
+      float nf;
+      fwd_rev(win5(dy_[1], dy_[2], dy_[3], dy_[4], dy_[5]), dy_[3], nf, yp);
     } else {
       yp = yplus[threadIdx.y + 1][threadIdx.x];
     }
@@ -430,22 +455,25 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
     if (active) {
       F r;
       if (RHS == kReinit) {
-        const F s0 = a.use_phi0 ? c0 : zw[3];
-        r = reinit_rhs(s0, a.use_phi0 != 0, xp, yp, zp, xm, ym, zm, a.dx_sq);
+        const F s0 = a.use_phi0 ? c0 : zw[0];
+        const float n2 = godunov_sq(s0 > 0.f, xp, yp, zp, xm, ym, zm, a.ix, a.iy, a.iz);
+        r = reinit_rhs(s0, a.use_phi0 != 0, n2, a.dx_sq);
       } else {
         const F v = RHS == kNormalField ? c0 : a.vn;
         r = 0.f;
         if (fabsf(v) >= kZeroTol)
-          r = r - v * __builtin_amdgcn_sqrtf(stencil::fastf::godunov_sq(v > 0.f, xp, yp, zp, xm, ym, zm));
+          r = r - v * __builtin_amdgcn_sqrtf(godunov_sq(v > 0.f, xp, yp, zp, xm, ym, zm, a.ix, a.iy, a.iz));
       }
-      const F uc = STAGE == 1 ? zw[3] : ucv;
-      a.out[off] = rk_combine<STAGE>(uc, zw[3], a.dt, r);
+      F uc = STAGE == 1 ? zw[0] : ucv;
+      asm volatile("" : "+v"(uc));  // (its product stays here, where the load is waited for anyway)
+      to_plane(a.out + zoff, own, rk_combine<STAGE>(uc, zw[0], a.dt, r));
     }
 #pragma unroll
-    for (int s = 0; s < 6; s++) zw[s] = zw[s + 1];
+    for (int s = 0; s < 3; s++) zw[s] = zw[s + 1];
 #pragma unroll
     for (int q = 0; q < 4; q++) dz[q] = dz[q + 1];
-  }
+  };
+  for (int k = kb; k <= ke; k++) step(k);
 }
 
 // ---------------------------------------------------------------------------

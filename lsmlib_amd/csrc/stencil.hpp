@@ -417,19 +417,22 @@ __device__ __forceinline__ float upwind(const float f[7], float inv, bool vpos) 
   return weno5(a, b, c, e, g) * inv;
 }
 
-// upwind() where the side taken is usually the same across a wave (a smooth
-// velocity): a wave whose lanes all take one side forms that side's window
-// alone, without a per-lane choice of operands.  Each lane's arithmetic is
-// that of upwind(), so a cell's result does not depend on the other lanes.
-__device__ __forceinline__ float upwind_wave(const float f[7], float inv, bool vpos) {
-  const unsigned long long pos = __builtin_amdgcn_ballot_w64(vpos), live = __builtin_amdgcn_ballot_w64(true);
+// upwind() by velocity, 0 where |vel| < tol, where the side taken is usually the
+// same across a wave (a smooth velocity): a wave whose lanes take one side forms
+// that side's window alone (the lanes below tol with it), without a per-lane
+// choice of operands.  Each lane's arithmetic is that of upwind(), so a cell's
+// result does not depend on the other lanes.
+__device__ __forceinline__ float upwind_wave(const float f[7], float inv, float vel, float tol) {
+  const bool on = !(fabsf(vel) < tol), vpos = vel > 0.f;
+  const unsigned long long pos = __builtin_amdgcn_ballot_w64(on && vpos);
+  const unsigned long long neg = __builtin_amdgcn_ballot_w64(on && !vpos);
   float d[6];
 #pragma unroll
   for (int s = -2; s <= 3; s++) d[s + 2] = f[s + 3] - f[s + 2];
   // (the empty asm keeps each side's arithmetic whole in its own branch; merged
   // tails would need register moves on every path)
   float r;
-  if (pos == live) {
+  if (neg == 0) {
     r = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[2]) * inv;
     asm volatile("" : "+v"(r));
   } else if (pos == 0) {
@@ -438,33 +441,33 @@ __device__ __forceinline__ float upwind_wave(const float f[7], float inv, bool v
   } else {
     r = upwind(f, inv, vpos);
   }
-  return r;
+  return on ? r : 0.f;
 }
 
 // Godunov |grad phi|^2 for a front that moves outward (pos) or inward, or for the
 // reinitialization on the side of sign pos: per axis the square of
 // max(m, -p, 0), or of max(-m, p, 0).  The signs are flipped by an exclusive or
 // and the larger is squared once (the squares' maximum is the maximum's square).
-__device__ __forceinline__ float godunov_sq(bool pos, float xp, float yp, float zp, float xm, float ym, float zm) {
+// The derivatives may come undivided, with the spacings' inverses.
+__device__ __forceinline__ float godunov_sq(bool pos, float xp, float yp, float zp, float xm, float ym, float zm,
+                                            float ix = 1.f, float iy = 1.f, float iz = 1.f) {
   const unsigned fm = pos ? 0u : 0x80000000u, fp = fm ^ 0x80000000u;
-  const float gp[3] = {xp, yp, zp}, gm[3] = {xm, ym, zm};
+  const float gp[3] = {xp, yp, zp}, gm[3] = {xm, ym, zm}, inv[3] = {ix, iy, iz};
   float n2 = 0.f;
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const float m = __uint_as_float(__float_as_uint(gm[d]) ^ fm), p = __uint_as_float(__float_as_uint(gp[d]) ^ fp);
-    const float st = fmaxf(fmaxf(m, p), 0.f);
+    const float st = fmaxf(fmaxf(m, p), 0.f) * inv[d];
     n2 = fmaf(st, st, n2);
   }
   return n2;
 }
 
 // Reinitialization RHS of one cell (the reference's formula,
-// lsm_reinitialization3d.f.in:167-199 and :251) with the hardware square root
-// and reciprocal square root (about 1 ulp each) in place of the correctly
-// rounded FP32 sqrt and division sequences.
-__device__ __forceinline__ float reinit_rhs(float s, bool use_phi0, float xp, float yp, float zp, float xm, float ym,
-                                            float zm, float dx_sq) {
-  const float n2 = godunov_sq(s > 0.f, xp, yp, zp, xm, ym, zm);
+// lsm_reinitialization3d.f.in:167-199 and :251) from its Godunov |grad phi|^2, with
+// the hardware square root and reciprocal square root (about 1 ulp each) in place
+// of the correctly rounded FP32 sqrt and division sequences.
+__device__ __forceinline__ float reinit_rhs(float s, bool use_phi0, float n2, float dx_sq) {
   if (!(fabsf(s) >= kZeroTol)) return 0.f;
   const float sgn = s * __builtin_amdgcn_rsqf(fmaf(s, s, use_phi0 ? dx_sq : n2 * dx_sq));
   return sgn * (1.f - __builtin_amdgcn_sqrtf(n2));
