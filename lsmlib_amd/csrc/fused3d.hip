@@ -939,22 +939,29 @@ int g_kchunk = 0;
 // (filling the z window, the launch of the block), so long chunks are cheaper
 // per plane; but a grid has to be cut into enough blocks to fill 256 CUs with
 // 2-4 resident blocks each, and into enough more that the last round of blocks
-// does not leave the chip idle.  The rule: chunks of at most 32 planes, shorter
-// where they would give fewer than kBlocks blocks, evened out over the planes.
+// does not leave the chip idle.  FP32: 32 planes where that gives 8192 blocks, 16
+// where it gives 2048, else at most 8, and fewer where they would give less than
+// 1024.  FP64 (blocks run 2-3 times longer per plane and fewer fit a CU, so the
+// tail weighs more): at most 32, fewer where they would give less than 2048.  The
+// chunks are evened out over the planes.
 // Measured (stage 2, us; chunks of 64 planes -> this rule): FP32 advection 64^3
-// 71.6 -> 5.7, 128^3 71 -> 16, 256^3 103 -> 82, 512^3 680 -> 672; FP64 advection
-// 64^3 201 -> 10, 128^3 160 -> 45, 203 x 149 x 97 212 -> 92, 512^3 2193 -> 2192.
-// FP64 blocks run 2-3 times longer per plane and fewer fit a CU, so the tail of
-// a short last round weighs more: twice the blocks.  Over 14 sizes from 32^3 to
-// 512^3 the rule is within 3 % (mean) of the best chunk of a sweep; 16 and 64
-// planes at most, and 512 blocks, were 1-4 % behind it.
+// 71.6 -> 5.7, 128^3 71 -> 16, 200^3 106 -> 54, 256^3 103 -> 79, 512^3 680 -> 672;
+// FP64 advection 64^3 201 -> 10, 128^3 160 -> 45, 203 x 149 x 97 212 -> 91, 512^3
+// 2193 -> 2192.  Over sizes from 32^3 to 512^3 the rules are within 3 % (mean) of
+// the best chunk of a sweep.
 int chunk_planes(const Box& fb, int nti, int ntj) {
-  constexpr long long kBlocks = sizeof(real_t) == 4 ? 1024 : 2048;
-  constexpr int kMost = 32;
   const int nz = fb.nz();
-  const long long fit = (long long)nti * ntj * nz / kBlocks;
-  const int kc = fit < 1 ? 1 : fit > kMost ? kMost : (int)fit;
-  const int chunks = (nz + kc - 1) / kc;
+  const long long tiles = (long long)nti * ntj, planes = tiles * nz;
+  long long kc;
+  if (sizeof(real_t) == 4) {
+    if (planes >= 32 * 8192LL) kc = 32;
+    else if (planes >= 16 * 2048LL) kc = 16;
+    else kc = planes / 1024 < 8 ? planes / 1024 : 8;
+  } else {
+    kc = planes / 2048 < 32 ? planes / 2048 : 32;
+  }
+  if (kc < 1) kc = 1;
+  const int chunks = (int)((nz + kc - 1) / kc);
   return (nz + chunks - 1) / chunks;
 }
 
