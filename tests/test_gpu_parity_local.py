@@ -37,6 +37,27 @@ def test_local_bitwise(hip, sym):
     H.assert_same(a, b, sym, out_abs=1e-13 if sym in SUMS else None)
 
 
+# What the level-0 points read where the lists end early: the differences that D1 held before the call, of every axis.
+@pytest.mark.parametrize("last", ["level 3", "level 2", "level 1", "level 0", "half of level 0", "none"])
+@pytest.mark.parametrize("mark_d1", [126, 124, 3, 1])
+def test_weno5_local_reads_what_d1_held(hip, last, mark_d1):
+    """Bands whose D1 lists stop at each level, inside level 0 and before it, with the 'big' value at the outer marks,
+    at the levels above a mark and almost everywhere: derivatives and D1 bitwise the oracle's, twice in a row (the
+    second call finds the first's D1)."""
+    sym = "lsm3dhjweno5local_"
+    c = _local_case(level=3, seed=4)
+    ends = {"level %d" % l: c.scalars["nhi%d" % l] for l in range(4)}
+    ends.update({"half of level 0": c.scalars["nhi0"] // 2, "none": c.scalars["nlo0"] - 1})
+    c.scalars["nhi3"] = ends[last]
+    c.scalars["mark_D1"] = mark_d1
+    for _ in range(2):
+        a = H.run(H.oracle(), sym, c)
+        b = H.run(hip.api, sym, c, device="cuda")
+        hip.check()
+        H.assert_same(a, b, sym)
+        c.arrays["D1"] = a[0]["D1"]
+
+
 @pytest.mark.parametrize("level", [1, 3, 4])
 @pytest.mark.parametrize("seed", [0, 1])
 def test_determine_narrow_band_bitwise(hip, level, seed):
