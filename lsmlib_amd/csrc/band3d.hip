@@ -31,10 +31,18 @@ static_assert(3 * kPer <= 64, "level-0 flags of a thread are kept in one 64-bit 
 constexpr int kChunk = kT * kPer;      // items per block
 constexpr int kNoClaim = 0x7fffffff;
 
-__device__ __forceinline__ int wave_prefix(bool f, int* total) {
+// Lanes before this one with f set.
+__device__ __forceinline__ int lane_prefix(bool f) {
   const unsigned long long m = __ballot(f);
-  *total = __popcll(m);
   return __popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull));
+}
+// Sum of x over this lane and those before it.
+__device__ __forceinline__ int wave_inclusive(int x) {
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if ((int)(threadIdx.x & 63) >= o) x += y;
+  }
+  return x;
 }
 
 // ----- level 0 ------------------------------------------------------------------------------------
@@ -66,42 +74,31 @@ struct Level0 {
   }
 };
 
-// Per-block placement of up to three flags over kPer passes of kT items
-// (item of pass it and thread x: base + it * kT + x).  Pass 1 loads and flags
-// every item, and each wave's count per pass and flag goes to LDS; after one
-// barrier, pass 2 places the items of each pass in item order: the block
-// offset is the counts of the earlier passes and of the earlier waves of the
-// same pass, plus the lane's prefix within its wave (a ballot).
+// Per-block placement of three flags over kPer passes of kT items (item of pass
+// it and thread x: base + it * kT + x).  Each wave's count per pass and flag
+// goes to LDS (record_pass), one wave per flag turns the 64 counts into offsets
+// (scan_passes), and an item's place is its wave's offset in its pass plus the
+// lane's prefix (a ballot).
 struct PassCounts {
-  int c[kPer][kT / 64][3];
+  int c[kPer * (kT / 64)][3];
 };
+static_assert(kPer * (kT / 64) == 64, "one lane per pass and wave");
 __device__ __forceinline__ void record_pass(PassCounts& pc, int it, const bool f[3]) {
   const int w = threadIdx.x >> 6;
 #pragma unroll
   for (int q = 0; q < 3; q++) {
     const int tot = __popcll(__ballot(f[q]));
-    if ((threadIdx.x & 63) == 0) pc.c[it][w][q] = tot;
+    if ((threadIdx.x & 63) == 0) pc.c[it * (kT / 64) + w][q] = tot;
   }
 }
-// Block offsets of this thread's items of pass it (flags f) given the totals
-// of the passes before it (run, advanced past pass it on return).  Every lane
-// of the wave must call it (it ballots).
-__device__ __forceinline__ void place_pass(const PassCounts& pc, int it, const bool f[3], int run[3], int off[3]) {
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    int tot;
-    const int lane_pre = wave_prefix(f[q], &tot);
-    int before = 0, all = 0;
-#pragma unroll
-    for (int v = 0; v < kT / 64; v++) {
-      const int x = pc.c[it][v][q];
-      before += v < w ? x : 0;
-      all += x;
-    }
-    off[q] = run[q] + before + lane_pre;
-    run[q] += all;
+__device__ __forceinline__ void scan_passes(PassCounts& pc) {
+  __syncthreads();
+  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (q < 3) {
+    const int x = pc.c[lane][q];
+    pc.c[lane][q] = wave_inclusive(x) - x;
   }
+  __syncthreads();
 }
 
 __global__ void __launch_bounds__(kT) level0_count_kernel(Level0 a, int* counts) {
@@ -180,6 +177,10 @@ struct Level0Out {
   Box nbb;
 };
 
+// Bound by VALU issue before the offsets came from one scan (each thread summed
+// the counts of every pass, 1280 VALU instructions a wave) and passes without a
+// band point placed none: a 512^3 FP32 grid, 303 -> 237 us; the field once and
+// the marks and lists out take 112.
 __global__ void __launch_bounds__(kT) level0_write_kernel(Level0 a, const int* offsets, Level0Out o) {
   __shared__ PassCounts pc;
   const long long base = (long long)blockIdx.x * kChunk;
@@ -197,8 +198,8 @@ __global__ void __launch_bounds__(kT) level0_write_kernel(Level0 a, const int* o
       for (int q = 0; q < 3; q++) fl |= (unsigned long long)f[q] << (3 * it + q);
     }
   }
-  __syncthreads();
-  int run[3] = {offsets[3 * blockIdx.x], offsets[3 * blockIdx.x + 1], offsets[3 * blockIdx.x + 2]};
+  scan_passes(pc);
+  const int first[3] = {offsets[3 * blockIdx.x], offsets[3 * blockIdx.x + 1], offsets[3 * blockIdx.x + 2]};
   // (i, j, k) of the thread's first cell, then advanced by kT cells per pass:
   // one division per thread instead of three per cell
   int i = a.B.ilo + (int)(t0 % a.nx);
@@ -210,13 +211,17 @@ __global__ void __launch_bounds__(kT) level0_write_kernel(Level0 a, const int* o
     const long long t = t0 + it * kT;
     const bool f[3] = {((fl >> (3 * it)) & 1ull) != 0, ((fl >> (3 * it + 1)) & 1ull) != 0,
                        ((fl >> (3 * it + 2)) & 1ull) != 0};
-    int off[3];
-    place_pass(pc, it, f, run, off);
     if (t < a.n) {
       const long long nbo = same ? t
                                  : (long long)(i - o.nbb.ilo) +
                                        (long long)o.nbb.nx() * ((j - o.nbb.jlo) + (long long)o.nbb.ny() * (k - o.nbb.klo));
       o.nb[nbo] = f[0] ? 1 : 0;
+    }
+    if (__any(f[0])) {
+      const int* before = pc.c[it * (kT / 64) + (threadIdx.x >> 6)];
+      int off[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) off[q] = first[q] + before[q] + lane_prefix(f[q]);
       if (f[0]) {
         const int r = off[0];
         o.ix[r] = i;
@@ -242,134 +247,145 @@ struct Grow {
   const int *ix, *iy, *iz;  // element 0 is index base; iz null for a 2D band
   int base;
   int plo;                  // first parent index
-  long long ncand;          // directions (6 in 3D, 4 in 2D) x parents
+  long long np;             // parents
   unsigned char* nb;
   Box nbb;
   int* claim;               // over nbb
-  unsigned char* win;       // per candidate: tried to claim a free cell (claim pass), then won it (count pass)
+  unsigned char* win;       // per parent, bit d: tried to claim a free cell (claim pass), then won it (count pass)
 };
+constexpr int kParents = 4;             // per thread of the count and write passes: one word of win
+constexpr int kParentChunk = kT * kParents;
 
-// NDIR (6 in 3D, 4 in 2D) is a template argument, so the candidate's split
-// into (parent, direction) is a division by a constant.
-template <int NDIR>
-__device__ __forceinline__ bool target(const Grow& g, long long c, int& off, int& qi, int& qj, int& qk, int* flag) {
-  if (c >= g.ncand) return false;
-  const int m = g.plo + (int)(c / NDIR), d = (int)(c % NDIR);
-  const int i = g.ix[m - g.base], j = g.iy[m - g.base], k = g.iz ? g.iz[m - g.base] : 0;
+// Few parents reach a free cell (of level 0, those at its surface), so what the
+// passes after the claims read of the others is one byte each: FP32, 10.1 M
+// level-0 points of a 512^3 grid, 1.4 M to each level: claim, count and write of
+// three levels 900 us with a byte per candidate, 604 so.
+
+// The cells next to a parent along +x, -x, +y, -y, +z, -z (candidate NDIR *
+// parent + direction): own offset and the steps.
+struct Near {
+  int o, step[6];
+};
+__device__ __forceinline__ Near near_cells(const Grow& g, int i, int j, int k) {
   const Box& b = g.nbb;
-  if (!b.has(i, j, k)) {
-    *flag = 1;
-    return false;
-  }
-  qi = i;
-  qj = j;
-  qk = k;
-  switch (d) {
-    case 0: if (!(i < b.ihi)) return false; qi = i + 1; break;
-    case 1: if (!(i > b.ilo)) return false; qi = i - 1; break;
-    case 2: if (!(j < b.jhi)) return false; qj = j + 1; break;
-    case 3: if (!(j > b.jlo)) return false; qj = j - 1; break;
-    case 4: if (!(k < b.khi)) return false; qk = k + 1; break;
-    default: if (!(k > b.klo)) return false; qk = k - 1; break;
-  }
-  off = (qi - b.ilo) + b.nx() * ((qj - b.jlo) + b.ny() * (qk - b.klo));
-  return true;
+  const int sy = b.nx(), sz = b.nx() * b.ny();
+  return Near{(i - b.ilo) + sy * ((j - b.jlo) + b.ny() * (k - b.klo)), {1, -1, sy, -sy, sz, -sz}};
 }
 
 // One thread per parent: its index read once, the marks of its NDIR
-// neighbours loaded together, then a claim for each free one (candidate
-// NDIR * parent + direction, as target() numbers them).
+// neighbours loaded together, then a claim for each free one.
 template <int NDIR>
 __global__ void __launch_bounds__(kT) claim_kernel(Grow g, int* flag) {
   const long long p = (long long)blockIdx.x * kT + threadIdx.x;
-  if (p >= g.ncand / NDIR) return;
+  if (p >= g.np) return;
   const long long c0 = NDIR * p;
   const int m = g.plo + (int)p;
   const int i = g.ix[m - g.base], j = g.iy[m - g.base], k = g.iz ? g.iz[m - g.base] : 0;
   const Box& b = g.nbb;
   if (!b.has(i, j, k)) {
     *flag = 1;
-#pragma unroll
-    for (int d = 0; d < NDIR; d++) g.win[c0 + d] = 0;
+    g.win[p] = 0;
     return;
   }
   const bool ok[6] = {i < b.ihi, i > b.ilo, j < b.jhi, j > b.jlo, k < b.khi, k > b.klo};
-  const int sy = b.nx(), sz = b.nx() * b.ny();
-  const int o = (i - b.ilo) + sy * ((j - b.jlo) + b.ny() * (k - b.klo));
-  const int step[6] = {1, -1, sy, -sy, sz, -sz};
+  const Near c = near_cells(g, i, j, k);
   unsigned char mk[NDIR];
 #pragma unroll
-  for (int d = 0; d < NDIR; d++) mk[d] = ok[d] ? g.nb[o + step[d]] : 1;
+  for (int d = 0; d < NDIR; d++) mk[d] = ok[d] ? g.nb[c.o + c.step[d]] : 1;
+  unsigned tried = 0;
 #pragma unroll
-  for (int d = 0; d < NDIR; d++) {
-    const bool tried = ok[d] && mk[d] == 0;
-    if (tried) atomicMin(&g.claim[o + step[d]], (int)(c0 + d));
-    g.win[c0 + d] = tried ? 1 : 0;  // the count pass looks only at these
+  for (int d = 0; d < NDIR; d++)
+    if (mk[d] == 0) {
+      atomicMin(&g.claim[c.o + c.step[d]], (int)(c0 + d));
+      tried |= 1u << d;
+    }
+  g.win[p] = (unsigned char)tried;
+}
+
+// The win bytes of parents p..p+3 (p a multiple of 4), 0 past the last.
+__device__ __forceinline__ unsigned win_word(const Grow& g, long long p) {
+  if (p >= g.np) return 0;
+  const unsigned w = *reinterpret_cast<const unsigned*>(g.win + p);
+  return p + kParents <= g.np ? w : w & ((1u << (8 * (int)(g.np - p))) - 1u);
+}
+// (i, j, k) of the parents of p..p+3 whose byte of w is not 0.
+__device__ __forceinline__ void load_parents(const Grow& g, long long p, unsigned w, int i[], int j[], int k[]) {
+#pragma unroll
+  for (int u = 0; u < kParents; u++) {
+    const long long m = g.plo - g.base + p + u;
+    i[u] = j[u] = k[u] = 0;
+    if ((w >> (8 * u)) & 255u) {
+      i[u] = g.ix[m];
+      j[u] = g.iy[m];
+      if (g.iz) k[u] = g.iz[m];
+    }
   }
 }
 
 template <int NDIR>
-__global__ void __launch_bounds__(kT) grow_count_kernel(Grow g, int* counts, int* flag) {
-  const long long base = (long long)blockIdx.x * kChunk;
-  int c = 0;
-  for (int it = 0; it < kPer; it++) {
-    const long long cand = base + it * kT + threadIdx.x;
-    // only candidates that tried to claim a free cell can have won it
-    bool w = false;
-    if (cand < g.ncand && g.win[cand]) {
-      int off, qi, qj, qk;
-      w = target<NDIR>(g, cand, off, qi, qj, qk, flag) && g.claim[off] == (int)cand;
-      g.win[cand] = w ? 1 : 0;
+__global__ void __launch_bounds__(kT) grow_count_kernel(Grow g, int* counts) {
+  const long long p = (long long)blockIdx.x * kParentChunk + (long long)threadIdx.x * kParents;
+  const unsigned tried = win_word(g, p);
+  int n = 0;
+  if (tried) {
+    int i[kParents], j[kParents], k[kParents];
+    load_parents(g, p, tried, i, j, k);
+    int owner[kParents][NDIR];
+#pragma unroll
+    for (int u = 0; u < kParents; u++) {
+      const Near c = near_cells(g, i[u], j[u], k[u]);
+#pragma unroll
+      for (int d = 0; d < NDIR; d++) owner[u][d] = (tried >> (8 * u + d)) & 1u ? g.claim[c.o + c.step[d]] : kNoClaim;
     }
-    c += w;
+    unsigned won = 0;
+#pragma unroll
+    for (int u = 0; u < kParents; u++)
+#pragma unroll
+      for (int d = 0; d < NDIR; d++)
+        if (owner[u][d] == (int)(NDIR * (p + u) + d)) won |= 1u << (8 * u + d);
+    *reinterpret_cast<unsigned*>(g.win + p) = won;
+    n = __popc(won);
   }
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
   __shared__ int s[kT / 64];
-  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = c;
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = n;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int v = 0; v < kT / 64; v++) t += s[v];
-    counts[3 * blockIdx.x] = t;
-    counts[3 * blockIdx.x + 1] = 0;
-    counts[3 * blockIdx.x + 2] = 0;
+  if (threadIdx.x < 3) {  // the scan takes triples
+    for (int v = 1; v < kT / 64; v++) n += s[v];
+    counts[3 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? n : 0;
   }
 }
 
+// Winners in candidate order: the parents of a thread follow each other, and
+// so do a parent's directions.
 template <int NDIR>
 __global__ void __launch_bounds__(kT) grow_write_kernel(Grow g, const int* offsets, int* ox, int* oy, int* oz,
-                                                        int start_rel, unsigned char mark, int* flag) {
-  __shared__ PassCounts pc;
-  const long long base = (long long)blockIdx.x * kChunk;
-  const long long c0 = base + threadIdx.x;
-  unsigned wins = 0;  // bit it: the count pass's result for pass it, all loaded first
-  {
-    unsigned char wb[kPer];
-#pragma unroll
-    for (int it = 0; it < kPer; it++) wb[it] = c0 + it * kT < g.ncand ? g.win[c0 + it * kT] : 0;
-#pragma unroll
-    for (int it = 0; it < kPer; it++) {
-      const bool f[3] = {wb[it] != 0, false, false};
-      record_pass(pc, it, f);
-      wins |= (unsigned)(wb[it] != 0) << it;
-    }
-  }
+                                                        int start_rel, unsigned char mark) {
+  const long long p = (long long)blockIdx.x * kParentChunk + (long long)threadIdx.x * kParents;
+  const unsigned won = win_word(g, p);
+  const int c = __popc(won), upto = wave_inclusive(c);
+  __shared__ int s[kT / 64];
+  if ((threadIdx.x & 63) == 63) s[threadIdx.x >> 6] = upto;
   __syncthreads();
-  int run[3] = {offsets[3 * blockIdx.x], 0, 0};
-  for (int it = 0; it < kPer; it++) {
-    const bool f[3] = {((wins >> it) & 1u) != 0, false, false};
-    int off[3];
-    place_pass(pc, it, f, run, off);
-    if (!f[0]) continue;
-    const long long cand = c0 + it * kT;
-    int off_cell = 0, qi = 0, qj = 0, qk = 0;
-    if (!target<NDIR>(g, cand, off_cell, qi, qj, qk, flag)) continue;  // cannot happen for a winner
-    const int r = start_rel + off[0];
-    ox[r] = qi;
-    oy[r] = qj;
-    if (oz) oz[r] = qk;
-    g.nb[off_cell] = mark;
-    g.claim[off_cell] = kNoClaim;
+  if (!won) return;
+  int r = start_rel + offsets[3 * blockIdx.x] + upto - c;
+  for (int w = 0; w < (int)(threadIdx.x >> 6); w++) r += s[w];
+  int i[kParents], j[kParents], k[kParents];
+  load_parents(g, p, won, i, j, k);
+#pragma unroll
+  for (int u = 0; u < kParents; u++) {
+    const Near n = near_cells(g, i[u], j[u], k[u]);
+#pragma unroll
+    for (int d = 0; d < NDIR; d++) {
+      if (!((won >> (8 * u + d)) & 1u)) continue;
+      const int cell = n.o + n.step[d];
+      ox[r] = i[u] + (d == 0) - (d == 1);
+      oy[r] = j[u] + (d == 2) - (d == 3);
+      if (oz) oz[r] = k[u] + (d == 4) - (d == 5);
+      g.nb[cell] = mark;
+      g.claim[cell] = kNoClaim;
+      r++;
+    }
   }
 }
 
@@ -427,7 +443,6 @@ bool grow_levels(const char* who, unsigned char* nb, const Box& nbb, int* ix, in
   const int ndir = iz ? 6 : 4;
   if (level < 1) return true;
   const long long ncells = nbb.volume();
-  long long maxcand = 0;
   if (!ensure(who, ncells, 1)) return false;
   int* flag = device_flag();
   if (!flag) return false;
@@ -440,18 +455,16 @@ bool grow_levels(const char* who, unsigned char* nb, const Box& nbb, int* ix, in
       continue;
     }
     const long long parents = (long long)n_hi[L - 1] - n_lo[L - 1] + 1;
-    const long long ncand = ndir * parents;
-    const long long nblk = (ncand + kChunk - 1) / kChunk;
-    if (ncand > maxcand) maxcand = ncand;
-    if (!ensure(who, ncells, nblk) || !ensure_win(who, ncand)) return false;
-    Grow g{ix, iy, iz, nlo, n_lo[L - 1], ncand, nb, nbb, g_claim, g_win};
+    const long long nblk = (parents + kParentChunk - 1) / kParentChunk;
+    if (!ensure(who, ncells, nblk) || !ensure_win(who, (parents + kParents - 1) / kParents * kParents)) return false;
+    Grow g{ix, iy, iz, nlo, n_lo[L - 1], parents, nb, nbb, g_claim, g_win};
     const dim3 cgrid((unsigned)((parents + kT - 1) / kT));  // one thread per parent
     if (ndir == 6) {
       hipLaunchKernelGGL(claim_kernel<6>, cgrid, dim3(kT), 0, stream(), g, flag);
-      hipLaunchKernelGGL(grow_count_kernel<6>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts, flag);
+      hipLaunchKernelGGL(grow_count_kernel<6>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts);
     } else {
       hipLaunchKernelGGL(claim_kernel<4>, cgrid, dim3(kT), 0, stream(), g, flag);
-      hipLaunchKernelGGL(grow_count_kernel<4>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts, flag);
+      hipLaunchKernelGGL(grow_count_kernel<4>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts);
     }
     hipLaunchKernelGGL(scan3_kernel, dim3(1), dim3(1024), 0, stream(), g_counts, nblk, g_tot);
     long long tot[3];
@@ -468,10 +481,10 @@ bool grow_levels(const char* who, unsigned char* nb, const Box& nbb, int* ix, in
     }
     if (ndir == 6)
       hipLaunchKernelGGL(grow_write_kernel<6>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts, ix, iy, iz,
-                         next - nlo, (unsigned char)(L + 1), flag);
+                         next - nlo, (unsigned char)(L + 1));
     else
       hipLaunchKernelGGL(grow_write_kernel<4>, dim3((unsigned)nblk), dim3(kT), 0, stream(), g, g_counts, ix, iy, iz,
-                         next - nlo, (unsigned char)(L + 1), flag);
+                         next - nlo, (unsigned char)(L + 1));
     if (!check_hip(hipGetLastError(), who)) return false;
     n_lo[L] = next;
     n_hi[L] = next + (int)tot[0] - 1;

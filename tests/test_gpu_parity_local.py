@@ -96,6 +96,35 @@ def test_determine_narrow_band_with_a_wider_mark_array(hip, level):
     assert (a[0]["nb"] == 9).sum() > 0
 
 
+# Around the 4 parents of a thread, the 1024 of a block, a wave's 64 x 4 and a level-0 chunk of 4096 cells.
+@pytest.mark.parametrize("points", [1, 2, 3, 4, 5, 255, 257, 1023, 1024, 1025, 4099])
+def test_band_grown_from_scattered_points(hip, points):
+    """Level 0 of a given number of scattered cells (each its own neighbourhood, some on the box's sides, some next to
+    each other and claiming the same cells), an outer layer of both signs, three levels: lists, outer list and marks
+    bitwise the oracle's."""
+    c = H.band_case(level=3, seed=6)
+    phi = c.arrays["phi"]
+    assert phi.size > 2 * 4099
+    rng = np.random.default_rng(points)
+    cells = rng.choice(phi.size, points, replace=False)
+    field = np.full(phi.size, 10.0 * c.scalars["width"])
+    field[cells] = rng.uniform(-1, 1, points) * c.scalars["width"]
+    phi[...] = field.reshape(phi.shape)
+    c.arrays["nb"] = np.full(H.shape_of(c.boxes["nb"]), 9, np.uint8)
+    for nm in ("ix", "iy", "iz", "outer"):
+        c.arrays[nm] = np.full(phi.size, -7, np.int32)
+    c.arrays["n_lo"] = np.full(4, -5, np.int32)
+    c.arrays["n_hi"] = np.full(4, -5, np.int32)
+    c.scalars.update(nlo=0, nhi=phi.size - 1, level=3)
+    sym = "lsm3ddeterminenarrowband_"
+    a = H.run(H.oracle(), sym, c)
+    b = H.run(hip.api, sym, c, device="cuda")
+    hip.check()
+    for k in ("nb", "ix", "iy", "iz", "outer", "n_lo", "n_hi"):
+        assert np.array_equal(a[0][k], b[0][k]), k
+    assert a[1] == b[1]
+
+
 def test_band_from_mask_and_outer_check(hip):
     for use_sign in (0, 1):
         c = _local_case(level=3)
