@@ -209,3 +209,37 @@ def test_stored_rhs_marks_points_whose_stencil_leaves_the_band():
     ha, hb = s.host(a), s.host(b)
     assert np.array_equal(ha, hb)
     assert (ha == 7.0).sum() > 0 and (ha != 7.0).sum() > 0
+
+
+def test_stage_and_dt_past_four_gigabytes(band):
+    """Fields whose byte offsets pass 2^32 at the band's points (the band's grid behind that many empty planes; the
+    marks keep their own box): the stage with its copies and the CFL step, bitwise those on the grid alone."""
+    r, vn = band
+    s, torch = r.solver, r.solver.torch
+    gb = list(r.grid.gb)
+    nz, ny, nx = r.phi.shape
+    extra = 2 ** 32 // (nx * ny * 8) + 1 - nz // 2  # the boundary lies inside the band's grid
+    far_gb = [ctypes.c_int(v) for v in gb[:4] + [gb[4] - extra, gb[5]]]
+    near, far = s._gb(), [ctypes.byref(v) for v in far_gb]
+    lo0, hi0, hi3 = int(r.n_lo[0]), int(r.n_hi[0]), int(r.n_hi[r.level])
+    ptrs = [b.data_ptr() for b in (r.ix, r.iy, r.iz)]
+    src = r.phi * 0.75 + 0.01
+    results = []
+    for box, off in ((near, 0), (far, extra)):
+        def field(values):
+            big = torch.empty((nz + off, ny, nx), dtype=s.dtype, device=s.device)
+            big[off:] = values
+            return big
+        us, uc, v, out = field(src), field(r.phi), field(vn), field(torch.full_like(r.phi, 7.0))
+        assert not off or us.numel() * 8 > 2 ** 32
+        dt = s.real(0)
+        s._ok(r._fdt(ctypes.byref(dt), us.data_ptr(), *box, 0.0, v.data_ptr(), *r.grid.dx, r.CFL, *ptrs, lo0, hi0,
+                     r.nb.data_ptr(), *near, r.MARKS[0], r.MARKS[2]))
+        s._ok(r._fstage(out.data_ptr(), us.data_ptr(), uc.data_ptr(), *box, 2, 0.0, v.data_ptr(), dt.value,
+                        *r.grid.dx, *ptrs, lo0, hi0, hi3, r.nb.data_ptr(), *near, r.MARKS[0], r.MARKS[2],
+                        r.width_inner, r.width))
+        s.lib.check()
+        results.append((dt.value, s.host(out[off:].contiguous())))
+        del us, uc, v, out
+    assert results[0][0] == results[1][0] > 0
+    assert np.array_equal(results[0][1], results[1][1])
