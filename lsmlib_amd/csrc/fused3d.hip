@@ -945,9 +945,9 @@ int g_kchunk = 0;
 // tail weighs more): at most 32, fewer where they would give less than 2048.  The
 // chunks are evened out over the planes.
 // Measured (stage 2, us; chunks of 64 planes -> this rule): FP32 advection 64^3
-// 71.6 -> 5.7, 128^3 71 -> 16, 200^3 106 -> 54, 256^3 103 -> 79, 512^3 680 -> 672;
-// FP64 advection 64^3 201 -> 10, 128^3 160 -> 45, 203 x 149 x 97 212 -> 91, 512^3
-// 2193 -> 2192.  Over sizes from 32^3 to 512^3 the rules are within 3 % (mean) of
+// 65.8 -> 5.4, 128^3 66 -> 16, 200^3 96 -> 52, 256^3 95 -> 75, 512^3 616 -> 600;
+// FP64 advection 64^3 181 -> 9.4, 128^3 137 -> 38, 203 x 149 x 97 185 -> 80, 512^3
+// 1789 -> 1776.  Over sizes from 32^3 to 512^3 the rules are within 3 % (mean) of
 // the best chunk of a sweep.
 int chunk_planes(const Box& fb, int nti, int ntj) {
   const int nz = fb.nz();
