@@ -168,7 +168,8 @@ int lsmhip_local_stage_from_rhs(LSMLIB_REAL *phi_out, const LSMLIB_REAL *phi_sta
  * given lam_out = dJ/d out on fb it adds b lam_out + (b dt dL/du_s)^T lam_out
  * to lam_us (ghost box), a lam_out to lam_uc (fb; unused for stage 1, may be
  * NULL) and -b dt sqrt(G) lam_out to lam_vn (fb; only with vn_field, may be
- * NULL).  scratch: 21 * |gb| reals.  Derivatives are those of the implemented
+ * NULL).  An array given for two or three of them takes the sum.  scratch:
+ * 21 * |gb| reals.  Derivatives are those of the implemented
  * WENO5/Godunov functions (argmax of the WENO eps, the selected Godunov branch). */
 int lsmhip_weno5_stage_normal_adjoint(LSMLIB_REAL *lam_us, LSMLIB_REAL *lam_uc, LSMLIB_REAL *lam_vn,
                                       const LSMLIB_REAL *lam_out, const LSMLIB_REAL *phi_stage, LSMHIP_BOX_ARGS(gb),

@@ -30,8 +30,10 @@
 //
 // adj_weights_kernel and adj_gather_kernel do the same through 21 weights per
 // cell in scratch.  They serve calls whose outputs overlap an input (the second
-// pass of the marches reads u_s again, after the first has written): pass 1
-// reads all inputs but lam_out, which pass 2 reads at its own cell.
+// pass of the marches reads u_s again, after the first has written: pass 1
+// reads all inputs but lam_out, which pass 2 reads at its own cell) or one
+// another (adj_coef_kernel reads all three before it writes any: each array is
+// added to by itself here, so one array takes the sum).
 //
 // Derivatives follow the implemented functions: the WENO5 weights
 // a_k = d_k/(S_k + eps)^2 with eps = 1e-6 max v^2 (the max contributes through
@@ -579,6 +581,7 @@ LSMHIP_EXPORT int lsmhip_weno5_stage_normal_adjoint(real_t* lam_us, real_t* lam_
   bool shared = false;
   for (const real_t* out : {A.lam_us, A.lam_uc, A.lam_v})
     for (const real_t* in : {A.us, A.lam_out, A.vnf}) shared = shared || overlap(out, in);
+  shared = shared || overlap(A.lam_us, A.lam_uc) || overlap(A.lam_us, A.lam_v) || overlap(A.lam_uc, A.lam_v);
   if (shared) {
     hipLaunchKernelGGL(adj_weights_kernel, grid_for(A.fb), block2d(), 0, stream(), A);
     hipLaunchKernelGGL(adj_gather_kernel, grid_for(A.gb), block2d(), 0, stream(), A);

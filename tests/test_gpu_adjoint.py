@@ -142,6 +142,34 @@ def test_stage_adjoint_over_tiles_and_sparse_gradients(n, share):
         assert d <= 1e-10 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("stage", [2, 3, 22])
+@pytest.mark.parametrize("one", ["us uc", "us v", "uc v", "us uc v"])
+def test_stage_adjoint_adds_up_in_one_array(stage, one):
+    """An array given for several of lam_us, lam_uc and lam_v (phi_stage and phi_n the same variable, say) holds what
+    it held plus all of their parts.  The two routes form the same terms in another order: 1e-10 of the largest, as
+    against autograd above."""
+    from lsmlib_amd.adjoint import NormalMotionAdjoint
+    from lsmlib_amd.solver import Grid
+    g = Grid((133, 101, 107))
+    eng = NormalMotionAdjoint(g, "f64", steps=1)
+    s = eng.solver
+    rng = np.random.default_rng(stage)
+    us, V, lam_out, was = (s.field(rng.standard_normal(g.shape)) for _ in range(4))
+    dt = 0.2 * min(g.dx)
+    own = {k: s.field() for k in ("us", "uc", "v")}
+    eng._stage_adjoint(own["us"], own["uc"], own["v"], lam_out, us, stage, V, dt)
+    both = was.clone()
+    out = {k: both if k in one.split() else s.field() for k in own}
+    eng._stage_adjoint(out["us"], out["uc"], out["v"], lam_out, us, stage, V, dt)
+    s.lib.check()
+    want = was + sum(own[k] for k in one.split())
+    scale = float(want.abs().max())
+    assert float((both - want).abs().max()) <= 1e-10 * scale
+    for k in own:
+        if k not in one.split():
+            assert float((out[k] - own[k]).abs().max()) <= 1e-10 * scale
+
+
 def test_two_forward_runs_on_one_engine_keep_their_own_gradients():
     """Two Evolve nodes on one engine before a single backward (a summed loss)
     give, for each speed and phi0, the gradients of separate runs: each node
