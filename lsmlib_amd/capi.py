@@ -362,7 +362,10 @@ def _addr(x):
 
 
 # Pointers to the ints of a box or of an integer argument, by value: a time loop
-# passes the same few boxes at every call, and the C side only reads them.  Given
+# passes the same few boxes at every call, and the C side only reads them.  Every
+# key is made of plain ints, so an argument that compares equal to one has its
+# value; what does not hash by value (a 0-d tensor, whose value may change between
+# two calls) or not at all (a 0-d array, a list) is converted at every call.  Given
 # up whole when a program has used more than _MOST different ones.
 _MOST = 4096
 _BOXES: dict = {}
@@ -370,19 +373,24 @@ _INTS: dict = {}
 
 
 def _box_pointers(box):
-    key = tuple(box)
-    ptrs = tuple(ctypes.byref(ctypes.c_int(int(v))) for v in key)
-    if len(_BOXES) >= _MOST:
-        _BOXES.clear()
-    _BOXES[key] = ptrs
+    key = tuple(int(v) for v in box)
+    ptrs = _BOXES.get(key)
+    if ptrs is None:
+        ptrs = tuple(ctypes.byref(ctypes.c_int(v)) for v in key)
+        if len(_BOXES) >= _MOST:
+            _BOXES.clear()
+        _BOXES[key] = ptrs
     return ptrs
 
 
 def _int_pointer(v):
-    ptr = ctypes.byref(ctypes.c_int(int(v)))
-    if len(_INTS) >= _MOST:
-        _INTS.clear()
-    _INTS[v] = ptr
+    key = int(v)
+    ptr = _INTS.get(key)
+    if ptr is None:
+        ptr = ctypes.byref(ctypes.c_int(key))
+        if len(_INTS) >= _MOST:
+            _INTS.clear()
+        _INTS[key] = ptr
     return ptr
 
 
@@ -412,11 +420,15 @@ class _Fn:
                     raise ValueError("box %s needs %d ints" % (name, 6 if kind == "B" else 4))
                 try:
                     ptrs = boxes[a]
-                except (KeyError, TypeError):  # a new box, or one that is no tuple
+                except (KeyError, TypeError):  # a new box, or one that is no tuple of ints
                     ptrs = _box_pointers(a)
                 cargs += ptrs
             elif kind == "S":
-                add(byref(real(a)))
+                try:
+                    c = real(a)
+                except TypeError:  # what float() alone takes (a text)
+                    c = real(float(a))
+                add(byref(c))
             elif kind == "I":
                 try:
                     add(ints[a])

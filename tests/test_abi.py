@@ -127,3 +127,34 @@ def test_binder_passes_each_call_its_own_values():
         assert got == [phi.ctypes.data, *gb, *fb, i, -0.0 if i % 5 else 0.5 * i, i % 256]
         assert math.copysign(1.0, got[12]) == (-1.0 if i % 5 else 1.0)
     assert len(capi._BOXES) <= capi._MOST and len(capi._INTS) <= capi._MOST
+
+
+def test_binder_converts_mutable_and_unhashable_arguments_at_each_call():
+    """A 0-d tensor (hashed by identity) passes the value it has at the call, as an integer and in a box; 0-d arrays
+    (no hash) are taken in both places; neither is kept alive.  A real scalar is what float() makes of it."""
+    import gc
+    import weakref
+
+    import torch
+    seen = []
+    fn = capi._Fn(lambda *a: seen.append([getattr(x, "_obj", x).value for x in a]),
+                  [("R", "phi"), ("Q", "gb"), ("I", "idx"), ("S", "dx")], ctypes.c_double)
+    phi = np.zeros(1)
+    for kind in (lambda v: torch.tensor(v), lambda v: np.array(v)):
+        i, c = kind(3), kind(5)
+        for box in ((c, 1, 2, 3), [c, 1, 2, 3]):
+            for v, w in ((3, 5), (4, 6), (-1, 7)):
+                i[...] = v
+                c[...] = w
+                fn(phi, box, i, "0.25")
+                assert seen.pop() == [phi.ctypes.data, w, 1, 2, 3, v, 0.25]
+    t = torch.tensor(3)
+    held = weakref.ref(t)
+    fn(phi, (t, 0, 0, 0), t, b"2.5")
+    assert seen.pop() == [phi.ctypes.data, 3, 0, 0, 0, 3, 2.5]
+    del t
+    gc.collect()
+    assert held() is None
+    for bad in ([1.0], None, "x"):
+        with pytest.raises((TypeError, ValueError)):
+            fn(phi, (0, 0, 0, 0), 0, bad)
