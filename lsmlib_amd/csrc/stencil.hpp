@@ -417,22 +417,20 @@ __device__ __forceinline__ float upwind(const float f[7], float inv, bool vpos) 
   return weno5(a, b, c, e, g) * inv;
 }
 
-// upwind() by velocity, 0 where |vel| < tol, where the side taken is usually the
-// same across a wave (a smooth velocity): a wave whose lanes take one side forms
-// that side's window alone (the lanes below tol with it), without a per-lane
-// choice of operands.  Each lane's arithmetic is that of upwind(), so a cell's
-// result does not depend on the other lanes.
-__device__ __forceinline__ float upwind_wave(const float f[7], float inv, float vel, float tol) {
-  const bool on = !(fabsf(vel) < tol), vpos = vel > 0.f;
-  const unsigned long long pos = __builtin_amdgcn_ballot_w64(on && vpos);
-  const unsigned long long neg = __builtin_amdgcn_ballot_w64(on && !vpos);
+// upwind() where the side taken is usually the same across a wave (a smooth
+// velocity): a wave whose lanes all take one side forms that side's window
+// alone, without a per-lane choice of operands.  Each lane's arithmetic is
+// that of upwind(); a cell's result depends on the other lanes only in which
+// products the compiler contracts.
+__device__ __forceinline__ float upwind_wave(const float f[7], float inv, bool vpos) {
+  const unsigned long long pos = __builtin_amdgcn_ballot_w64(vpos), live = __builtin_amdgcn_ballot_w64(true);
   float d[6];
 #pragma unroll
   for (int s = -2; s <= 3; s++) d[s + 2] = f[s + 3] - f[s + 2];
   // (the empty asm keeps each side's arithmetic whole in its own branch; merged
   // tails would need register moves on every path)
   float r;
-  if (neg == 0) {
+  if (pos == live) {
     r = fwd(win5(d[0], d[1], d[2], d[3], d[4]), d[2]) * inv;
     asm volatile("" : "+v"(r));
   } else if (pos == 0) {
@@ -441,7 +439,7 @@ __device__ __forceinline__ float upwind_wave(const float f[7], float inv, float 
   } else {
     r = upwind(f, inv, vpos);
   }
-  return on ? r : 0.f;
+  return r;
 }
 
 // Godunov |grad phi|^2 for a front that moves outward (pos) or inward, or for the

@@ -221,3 +221,44 @@ def test_fp64_advection_by_lane_is_bitwise_the_oracle(nx, signs):
     H.oracle().lsm3dupwindhjweno5(o[0], o[1], o[2], gb, phi, gb, *vel, gb, o[3], gb, fb, *g.dx)
     for a, b in zip(G[:3], o[:3]):
         assert np.array_equal(g.interior(s.host(a)), g.interior(b))
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("pattern", ["zero waves", "one lane", "mixed"])
+def test_fp32_advection_of_a_cell_does_not_depend_on_its_wave(axis, pattern):
+    """Speeds along one axis that are positive, negative, below the zero tolerance (both signs) or exactly zero: waves
+    without a speed, with one, and of every kind take different routes, and each cell has the value it has where all
+    speeds are of its own kind: without a speed the same bits; with one, the routes may contract different products, and
+    the derivative, bounded by the largest difference, moves by some 50 roundings (as above, four times for the
+    weights), of which dt |v| / dx enters."""
+    from lsmlib_amd.solver import Grid, Solver
+    g = Grid((130, 17, 9), hi=(1.3, 0.17, 0.09))
+    s = Solver(g, "f32")
+    rng = np.random.default_rng(axis)
+    phi, phin = (s.field(rng.standard_normal(g.shape)) for _ in range(2))
+    size = np.abs(rng.standard_normal(g.shape)) + 0.1
+    kind = rng.integers(-1, 2, g.shape)
+    if pattern == "zero waves":
+        kind[:, ::2, :] = 0
+        kind[:, :, :g.g + 64] = 0
+    elif pattern == "one lane":
+        kind[...] = 0
+        kind[:, :, g.g::64] = -1
+        kind[:, :, g.g + 63::64] = 1
+    tiny = np.where(rng.random(g.shape) < 0.5, rng.choice([-1e-16, 1e-16], g.shape), 0.0)
+
+    def stage(speed):
+        vel = [s.field() for _ in range(3)]
+        vel[axis] = s.field(speed)
+        out = s.field()
+        s.stage_advect(out, phi, phin, 3, 0.003, vel)
+        s.lib.check()
+        return g.interior(s.host(out))
+
+    got = stage(np.where(kind == 0, tiny, kind * size))
+    inner = g.interior(kind)
+    bound = 0.003 * size.max() / 0.01 * 4 * 50 * 2.0 ** -24 * 2 * float(phi.abs().max())
+    assert bound < 1e-3
+    for k in (-1, 0, 1):
+        d = np.abs(got - stage(k * size))[inner == k]
+        assert d.max() <= (bound if k else 0.0), k
