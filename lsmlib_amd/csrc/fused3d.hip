@@ -21,6 +21,8 @@
 // the FP64 build a stage is bitwise equal to
 //   HJ_WENO5 / UPWIND_HJ_WENO5 -> zero RHS -> add term -> TVD_RK3_STAGEn
 // of the reference on the same inputs.
+#include <initializer_list>
+
 #include "lsmhip_core.hpp"
 #include "stencil.hpp"
 
@@ -949,24 +951,43 @@ int g_kchunk = 0;
 // tail weighs more): at most 32, fewer where they would give less than 2048.  The
 // chunks are evened out over the planes.
 // Measured (stage 2, us; chunks of 64 planes -> this rule): FP32 advection 64^3
-// 65.8 -> 5.4, 128^3 66 -> 16, 200^3 96 -> 52, 256^3 95 -> 75, 512^3 616 -> 600;
+// 65.8 -> 5.4, 128^3 66 -> 16, 200^3 96 -> 52, 256^3 95 -> 73, 512^3 616 -> 550;
 // FP64 advection 64^3 181 -> 9.4, 128^3 137 -> 38, 203 x 149 x 97 185 -> 80, 512^3
-// 1789 -> 1776.  Over sizes from 32^3 to 512^3 the rules are within 3 % (mean) of
+// 1789 -> 1705.  Over sizes from 32^3 to 512^3 the rules are within 3 % (mean) of
 // the best chunk of a sweep.
+// A few planes over many tiles are the exception: the tiles alone fill the chip,
+// and cut into single planes they pay the fixed part for each.  There 2 or 4
+// planes are taken where that makes the rounds of 512 blocks times the planes and
+// half a plane (the fixed part) no more.  FP64 deformation advection, us, the rule
+// above -> so (and whole columns): 512 x 512 x 3 19.8 -> 14.1 (14.1), x 4
+// 23.7 -> 15.8 (15.8), x 6 33.3 -> 25.1 (23.3), x 8 36.7 -> 31.3 (30.9); 576 x 512
+// x 4 28.0 -> 22.1 (22.8); reinitialization x 4 32.7 -> 31.6, 576 x 512 x 4
+// 35.6 -> 39.1 (43.3); FP32 deformation x 3 10.8 -> 8.8, x 4 10.4 -> 10.0.  With 350
+// tiles whole columns are slower (reinitialization 400 x 400 x 4 25.6, 30.8).
 int chunk_planes(const Box& fb, int nti, int ntj) {
   const int nz = fb.nz();
   const long long tiles = (long long)nti * ntj, planes = tiles * nz;
-  long long kc;
+  long long fit;
   if (sizeof(real_t) == 4) {
-    if (planes >= 32 * 8192LL) kc = 32;
-    else if (planes >= 16 * 2048LL) kc = 16;
-    else kc = planes / 1024 < 8 ? planes / 1024 : 8;
+    if (planes >= 32 * 8192LL) fit = 32;
+    else if (planes >= 16 * 2048LL) fit = 16;
+    else fit = planes / 1024 < 8 ? planes / 1024 : 8;
   } else {
-    kc = planes / 2048 < 32 ? planes / 2048 : 32;
+    fit = planes / 2048 < 32 ? planes / 2048 : 32;
   }
-  if (kc < 1) kc = 1;
-  const int chunks = (int)((nz + kc - 1) / kc);
-  return (nz + chunks - 1) / chunks;
+  auto even = [&](int k) {
+    const int chunks = (nz + k - 1) / k;
+    return (nz + chunks - 1) / chunks;
+  };
+  int kc = even(fit < 1 ? 1 : (int)fit);
+  if (tiles >= 384 && nz <= 8) {
+    auto cost = [&](int k) { return (tiles * ((nz + k - 1) / k) + 511) / 512 * (2 * k + 1); };
+    for (const int most : {2, 4}) {
+      const int k = even(most);
+      if (k > kc && cost(k) <= cost(kc)) kc = k;
+    }
+  }
+  return kc;
 }
 
 int run(const char* who, FusedArgs a, int stage) {

@@ -262,3 +262,13 @@ def test_fp32_advection_of_a_cell_does_not_depend_on_its_wave(axis, pattern):
     for k in (-1, 0, 1):
         d = np.abs(got - stage(k * size))[inner == k]
         assert d.max() <= (bound if k else 0.0), k
+
+
+# A few planes over 384 tiles and more: 2, 3 and 4 planes a chunk, in one and in several rounds of 512 blocks, and the
+# sizes on either side of that rule.
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [(512, 384, 3), (449, 385, 4), (576, 512, 4), (512, 512, 6), (512, 384, 8), (512, 384, 9),
+                               (448, 432, 4)])
+def test_thin_grids_do_not_depend_on_the_chunks(prec, n):
+    test_stage_does_not_depend_on_the_chunks(prec, n, "reinit")
+    test_stage_does_not_depend_on_the_chunks(prec, n, "advect")
