@@ -221,3 +221,29 @@ def test_neumann_zero_normal_derivative_2d_hip(hip, scheme):
     I = (slice(3, -3),) * 2
     assert np.abs(a["pxm"][I][:, 0]).max() < 1e-6 and np.abs(a["pxp"][I][:, -1]).max() < 1e-6
     assert np.abs(a["pym"][I][0, :]).max() < 1e-6 and np.abs(a["pyp"][I][-1, :]).max() < 1e-6
+
+
+def test_f32_2d_weno5_does_not_depend_on_the_store_order(hip32):
+    """A fill box past the size from which each axis is stored when it is done, against its two halves, which are below
+    it: the same operations, of which the two kernels may contract others (some 50 roundings of the largest difference,
+    four times for the weights).  Rows of 64 q + 1 cells."""
+    import torch
+    nx, ny, h = 4097, 3900, 0.25
+    gb = (-3, nx + 2, -3, ny + 2)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    phi = torch.randn(ny + 6, nx + 6, device="cuda", generator=gen)
+    D1 = torch.zeros_like(phi)
+
+    def pm(parts):
+        out = [torch.zeros_like(phi) for _ in range(4)]
+        for fb in parts:
+            hip32.api.lsm2dhjweno5(out[0], out[1], gb, out[2], out[3], gb, phi, gb, D1, gb, fb, h, h)
+        hip32.check()
+        return out
+
+    whole = pm([(0, nx - 1, 0, ny - 1)])
+    halves = pm([(0, nx - 1, 0, ny // 2 - 1), (0, nx - 1, ny // 2, ny - 1)])
+    bound = 4 * 50 * 2.0 ** -24 * 2 * float(phi.abs().max()) / h
+    for a, b in zip(whole, halves):
+        assert float(a.abs().max()) > 1.0
+        assert float((a - b).abs().max()) <= bound
