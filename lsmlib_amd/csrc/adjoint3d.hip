@@ -33,7 +33,7 @@
 // pass of the marches reads u_s again, after the first has written: pass 1
 // reads all inputs but lam_out, which pass 2 reads at its own cell) or one
 // another (adj_coef_kernel reads all three before it writes any: each array is
-// added to by itself here, so one array takes the sum).
+// added to by itself here, so one array takes the sum), and small grids (marched).
 //
 // Derivatives follow the implemented functions: the WENO5 weights
 // a_k = d_k/(S_k + eps)^2 with eps = 1e-6 max v^2 (the max contributes through
@@ -526,6 +526,27 @@ __global__ void __launch_bounds__(256) mismatch_grad_kernel(real_t* grad, const 
   grad[o] = (real_t)g;
 }
 
+// The marches are chains of a memory round trip per cell, seven at the least, which
+// a small grid has too few columns to hide, while its 21 weights a cell lie in the
+// caches.  By the fill box's waves (rows cut into 64 cells), and by those that the
+// weights' kernels launch for them (rows in groups of 32: many more where there are
+// few rows along j); a stage, us, weights / marches, lam_out not zero within 4 cells
+// of an interface and everywhere:
+//   FP32 64^3 (4096 waves) 32 / 51, 37 / 56; 96^3 (18432) 59 / 63, 70 / 84; 104^3
+//   (21632) 73 / 71, 87 / 90; 112^3 (25088) 77 / 72, 94 / 111; 128^3 (32768) 120 / 82,
+//   133 / 126; 512 x 4 x 512 (16384, 131072 launched) 335 / 130 both
+//   FP64 64^3 40 / 68, 47 / 79; 96^3 89 / 111, 110 / 157; 60 x 90 x 200 (18000)
+//   113 / 124, 149 / 195; 104^3 124 / 126, 157 / 174; 60 x 120 x 200 (24000) 203 / 144,
+//   232 / 228; 112^3 169 / 147, 201 / 224; 120^3 (28800) 201 / 152, 236 / 246; 128^3
+//   266 / 163, 290 / 252
+// The line is drawn for gradients near an interface, which is what a loss of a level
+// set has.
+bool marched(const Box& f) {
+  const dim3 g = grid_for(f);
+  const long long waves = (long long)((f.nx() + 63) / 64) * f.ny() * f.nz();
+  return waves >= 24000 || (long long)g.x * g.y * g.z * kBY >= 32768;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -582,7 +603,7 @@ LSMHIP_EXPORT int lsmhip_weno5_stage_normal_adjoint(real_t* lam_us, real_t* lam_
   for (const real_t* out : {A.lam_us, A.lam_uc, A.lam_v})
     for (const real_t* in : {A.us, A.lam_out, A.vnf}) shared = shared || overlap(out, in);
   shared = shared || overlap(A.lam_us, A.lam_uc) || overlap(A.lam_us, A.lam_v) || overlap(A.lam_uc, A.lam_v);
-  if (shared) {
+  if (shared || !marched(A.fb)) {
     hipLaunchKernelGGL(adj_weights_kernel, grid_for(A.fb), block2d(), 0, stream(), A);
     hipLaunchKernelGGL(adj_gather_kernel, grid_for(A.gb), block2d(), 0, stream(), A);
     return finish(who) ? 0 : -1;

@@ -142,6 +142,80 @@ def test_stage_adjoint_over_tiles_and_sparse_gradients(n, share):
         assert d <= 1e-10 * np.abs(ref).max()
 
 
+def _well_conditioned(us, V, dx):
+    """Cells whose derivative hangs on no rounding: each of the six reconstructions has normalised smoothness terms of
+    0.01 or more, the Godunov sides of an axis differ, and |grad phi| does not vanish."""
+    import torch
+    ok = torch.ones_like(us, dtype=torch.bool)
+    G = 0
+    for dim, h in ((2, dx[0]), (1, dx[1]), (0, dx[2])):
+        f = {s: torch.roll(us, shifts=-s, dims=dim) for s in range(-3, 4)}
+        D = {t: (f[t] - f[t - 1]) / h for t in range(-2, 4)}
+        val = []
+        for v1, v2, v3, v4, v5 in ([D[3], D[2], D[1], D[0], D[-1]], [D[-2], D[-1], D[0], D[1], D[2]]):
+            m = torch.stack([x * x for x in (v1, v2, v3, v4, v5)]).amax(0)
+            S = [13 / 12 * (v1 - 2 * v2 + v3) ** 2 + 0.25 * (v1 - 4 * v2 + 3 * v3) ** 2,
+                 13 / 12 * (v2 - 2 * v3 + v4) ** 2 + 0.25 * (v2 - v4) ** 2,
+                 13 / 12 * (v3 - 2 * v4 + v5) ** 2 + 0.25 * (3 * v3 - 4 * v4 + v5) ** 2]
+            for x in S:
+                ok &= x >= 0.01 * m
+            a = [d / (x + 1e-6 * m) ** 2 for d, x in zip((0.1, 0.6, 0.3), S)]
+            p = (v1 / 3 - 7 * v2 / 6 + 11 * v3 / 6, -v2 / 6 + 5 * v3 / 6 + v4 / 3, v3 / 3 + 5 * v4 / 6 - v5 / 6)
+            val.append(sum(x * y for x, y in zip(a, p)) / sum(a))
+        A = torch.where(V > 0, val[1].clamp(min=0), val[1].clamp(max=0)) ** 2
+        B = torch.where(V > 0, val[0].clamp(max=0), val[0].clamp(min=0)) ** 2
+        ok &= ((A - B).abs() > 1e-3 * (A + B)) | (A + B == 0)
+        G = G + torch.maximum(A, B)
+    return ok & (G > 0.01 / max(dx) ** 2)
+
+
+# The marches serve fill boxes of 24000 waves (rows of 64 cells) and more.  Their tiles of 58 targets along x: one, one
+# full, one target past one and past two; chunks of 8 targets along j and k with a last one of a single target, and
+# long ones; the smallest periodic extents.
+@pytest.mark.parametrize("n", [(3, 155, 157), (52, 3, 8010), (53, 163, 150), (65, 66, 190), (111, 3, 4010), (117, 4010, 3)])
+@pytest.mark.parametrize("share", [0.0, 0.02, 1.0])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_stage_adjoint_marches(n, share, prec):
+    """Against torch autograd in FP64 on the same inputs.  A normalised smoothness term e moves by up to 50 roundings, a
+    weight by 100 / e of them, and a gradient by three of those: FP64, e >= 1e-6 (eps), 4e-8 of the largest; FP32, at
+    cells whose derivative hangs on no rounding, e >= 0.01: 2e-3."""
+    import torch
+    from lsmlib_amd.adjoint import NormalMotionAdjoint
+    from lsmlib_amd.solver import Grid
+    g = Grid(n, hi=tuple(0.02 * v for v in n))
+    eng = NormalMotionAdjoint(g, prec, steps=1)
+    s = eng.solver
+    gen = torch.Generator(device="cuda").manual_seed(n[0])
+    shape = (n[2], n[1], n[0])
+    us, uc, V, lam = (torch.randn(shape, generator=gen, device="cuda").to(s.dtype).double() for _ in range(4))
+    V = torch.where(V < 0, -1.0, 1.0) * (0.5 + V.abs())
+    V = V.to(s.dtype).double()
+    lam = torch.where(torch.rand(shape, generator=gen, device="cuda") < share, lam, 0.0)
+    if prec == "f32":
+        ok = _well_conditioned(us, V, g.dx)
+        assert float(ok.double().mean()) > 0.1
+        lam = torch.where(ok, lam, 0.0)
+    dt, stage = 0.004, 2
+    leaves = [t.clone().requires_grad_(True) for t in (us, uc, V)]
+    want = torch.autograd.grad((_torch_stage(*leaves, dt, g.dx, stage) * lam).sum(), leaves)
+
+    def ghost(t):
+        full = s.field()
+        g.interior(full)[...] = t.to(s.dtype)
+        return full
+
+    d_us, d_V, d_lam = ghost(us), ghost(V), ghost(lam)
+    s.fill_ghosts(d_us)
+    out = [s.field() for _ in range(3)]
+    eng._stage_adjoint(*out, d_lam, d_us, stage, d_V, dt)
+    eng._fold_ghosts(out[0])
+    s.lib.check()
+    for name, got, ref in zip(("phi_stage", "phi_n", "V"), out, want):
+        d = float((g.interior(got).double() - ref).abs().max())
+        print(name, d, float(ref.abs().max()))
+        assert d <= (4e-8 if prec == "f64" else 2e-3) * float(ref.abs().max()), name
+
+
 @pytest.mark.parametrize("stage", [2, 3, 22])
 @pytest.mark.parametrize("one", ["us uc", "us v", "uc v", "us uc v"])
 def test_stage_adjoint_adds_up_in_one_array(stage, one):
