@@ -425,10 +425,9 @@ class _Fn:
                 cargs += ptrs
             elif kind == "S":
                 try:
-                    c = real(a)
+                    add(byref(real(a)))
                 except TypeError:  # what float() alone takes (a text)
-                    c = real(float(a))
-                add(byref(c))
+                    add(byref(real(float(a))))
             elif kind == "I":
                 try:
                     add(ints[a])
