@@ -489,8 +489,8 @@ __global__ void __launch_bounds__(TX* TY) fused_pm_f32_kernel(FusedArgs a) {
 // Along an axis, write D(m) = u(m) - u(m-1) and, for the three consecutive
 // differences around position m, A(m) = D(m-1) - 2 D(m) + D(m+1),
 // C(m) = D(m-1) - D(m+1) and T(m) = 13/3 A(m)^2.  The minus-side
-// reconstruction at m, weno5(D(m-2), .., D(m+2)), needs (4 S_k = 13/3 a_k^2 +
-// b_k^2, the scaling of stencil::fastf::win5)
+// reconstruction at m, weno5(D(m-2), .., D(m+2)), needs (the indicators times 4,
+// and so eps = 4e-6 max D^2: 4 S_k = 13/3 a_k^2 + b_k^2)
 //   4 S1 = T(m-1) + (2 A(m-1) - C(m-1))^2,  4 S2 = T(m) + C(m)^2,
 //   4 S3 = T(m+1) + (2 A(m+1) + C(m+1))^2,
 //   a1 - a2 = A(m-1) - A(m),  a2 - a3 = A(m) - A(m+1),
@@ -902,10 +902,12 @@ __global__ void __launch_bounds__(TX* TY) fused_pm2_f32_kernel(FusedArgs a) {
 
 // FP32 stage kernels: 1 (default) = the per-cell window kernels
 // (fused_stage_kernel, fused_pm_f32_kernel), 2 = the shared-quantity kernels
-// (fused_advect_f32_kernel, fused_pm2_f32_kernel).  The second set issues
-// 14-20 % fewer VALU instructions per cell but holds 72-80 VGPRs and meets
-// four barriers per plane; at the 6 waves per SIMD that allows it runs slower
-// on gfx950 (0.91 vs 0.76 ms per 512^3 advection stage).  It stays as an
+// (fused_advect_f32_kernel, fused_pm2_f32_kernel).  Since the windows of the first set
+// take their indicators from second differences, the second issues more VALU
+// instructions for advection (190 a cell-stage, 182) and 5 % fewer for the
+// reinitialization (210, 221), holds 70-80 VGPRs and meets four barriers per plane;
+// at the 6 waves per SIMD that allows it runs slower on gfx950 (512^3 stage 2, traced:
+// advection 0.89 vs 0.63 ms, reinitialization 0.85 vs 0.69).  It stays as an
 // independent rounding order for precision comparisons.  FP64 always runs
 // fused_stage_kernel.
 int g_f32_kernels = 1;

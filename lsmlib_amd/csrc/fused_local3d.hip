@@ -54,7 +54,9 @@ struct LocalStage {
 // the point's own byte offset (load_cross), the box tests are one (make_stage),
 // and the marks are tested by their extremes (18 compares and 18 selects only in
 // a wave with a mark above mark_D1).  FP32, 10.1 M points of a 512^3 grid: stage
-// 3 166 -> 160 us, stage 2 268 -> 261, the CFL pass 147 -> 141.
+// 3 166 -> 160 us, stage 2 268 -> 261, the CFL pass 147 -> 141.  The stages hold 65
+// registers so (7 waves a SIMD; 56 and 8 with 64-bit addresses): held to 64 they
+// spill, and stage 3 takes 171 us, stage 2 272.
 __device__ __forceinline__ bool cross_in_boxes(const LocalStage& a, int i, int j, int k) {
   return (unsigned)i - (unsigned)a.clo[0] < a.cn[0] && (unsigned)j - (unsigned)a.clo[1] < a.cn[1] &&
          (unsigned)k - (unsigned)a.clo[2] < a.cn[2];

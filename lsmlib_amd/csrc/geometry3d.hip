@@ -290,7 +290,7 @@ struct Factors4 {
 // derivatives (:342-351): phi_xy = d/dy phi_x, phi_yz = d/dz phi_y,
 // phi_zx = d/dx phi_z.  GAUSS = 0: mean curvature over |grad phi|^3 (numerator
 // order of :358-366); GAUSS = 1: Gaussian curvature over |grad phi|^4.
-// On the plane march (64 x 8 tiles, chunks of 16 planes): phi with its x and
+// On the plane march (64 x 8 tiles, chunks by march::chunk_planes): phi with its x and
 // y neighbours, phi_x with its y neighbours and phi_z with its x neighbours
 // staged per plane in LDS (two-cell halos), phi and phi_y along z carried in
 // registers, every next-plane value in flight while the plane is computed.

@@ -344,7 +344,8 @@ __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x);
 // p3 - p2 = (a2 - a3)/6, p2 = v3 + t34/3 + t23/6,
 //   sum_k w_k p_k = p2 + (q23 (a1 - a2)/3 + q12 (a2 - a3)/2) / (q23 + 6 q13 + 3 q12).
 // 47 VALU instructions a derivative from its six values, 52 with S_k formed as
-// two squares each (VALU instructions a cell-stage: advection 185 -> 172, reinitialization 244 -> 224).
+// two squares each.  (A cell-stage at 512^3 with its 32-plane chunks' starts, about
+// 3: advection 182 VALU instructions, reinitialization 221.)
 struct Win {
   float q12, q13, q23, d12, d23, t23, t34;
 };
